@@ -22,7 +22,7 @@ CFLAGS_HOST := -O2 -fPIC -std=c11 -Wall -Wextra -D__HIP_PLATFORM_AMD__ -I$(ROCM)
 
 HOST_SRCS := $(CSRC)/runtime.c $(CSRC)/tensor.c $(CSRC)/ops.c $(CSRC)/autograd.c $(CSRC)/dataset.c
 HIP_SRCS  := $(CSRC)/gemm.hip $(CSRC)/conv.hip $(CSRC)/elementwise.hip $(CSRC)/spatial.hip \
-             $(CSRC)/head.hip
+             $(CSRC)/head.hip $(CSRC)/conv_gen.hip
 HDRS      := $(wildcard include/*.h) $(wildcard $(CSRC)/*.h)
 HOST_OBJS := $(patsubst $(CSRC)/%.c,$(BUILD)/obj/%.o,$(HOST_SRCS))
 HIP_OBJS  := $(patsubst $(CSRC)/%.hip,$(BUILD)/obj/%.o,$(HIP_SRCS))
@@ -43,7 +43,7 @@ $(BUILD)/obj/gemm.o: $(CSRC)/gemm.hip $(HDRS) | $(BUILD)/obj
 
 # direct convolution: MFMA accumulators in VGPRs (the AGPR form made the
 # compiler copy accumulators between register files every loop iteration)
-$(BUILD)/obj/conv.o: $(CSRC)/conv.hip $(HDRS) | $(BUILD)/obj
+$(BUILD)/obj/conv.o $(BUILD)/obj/conv_gen.o: $(BUILD)/obj/%.o: $(CSRC)/%.hip $(HDRS) | $(BUILD)/obj
 	$(HIPCC) $(HIPFLAGS) -ffp-contract=off -mllvm -amdgpu-mfma-vgpr-form=1 -c $< -o $@
 
 $(BUILD)/obj/%.o: $(CSRC)/%.hip $(HDRS) | $(BUILD)/obj

@@ -1201,18 +1201,21 @@ static void backward_conv2d(AGNode *n) {
     const int chained = conv_chain_bwd(n, gd);
     if (chained == 2) return;
     const long bshp[1] = {F};
-    const int lds = tt_k_conv2d_lds_plan(N, C, H, W, F, HH, WW, sh, sw, ph, pw, Ho, Wo);
+    const int q[13] = {N, C, H, W, F, HH, WW, sh, sw, ph, pw, Ho, Wo};
+    const int route_w = needs(w) && !n->at.conv.col ? ttk_conv_route(q, 1) : 0;
     int w_done = 0;
-    if (needs(w) && !n->at.conv.col && (lds & 2)) {
-        /* LDS-staged forward kept no col: dW (and db) read x */
+    if (route_w) {
+        /* the direct forward kept no col: dW (and db) read x */
         const float *x = tt_dev(a->val);
         Tensor *gw = x ? tt_empty_like(w->val) : NULL;
         Tensor *gb = gw && needs(b) ? tt_empty_dev(bshp, 1) : NULL;
-        const int q[13] = {N, C, H, W, F, HH, WW, sh, sw, ph, pw, Ho, Wo};
+        float *dbd = gb ? gb->dev : NULL;
         if (gw && (gb || !needs(b)) &&
-            (conv_dw_deferred(gd, NULL, x, gw, gb, q) == 0 ||
-             tt_k_conv2d_dw_lds(gd, x, gw->dev, gb ? gb->dev : NULL, N, C, H, W, F, HH, WW, sh,
-                                sw, ph, pw, Ho, Wo) == 0)) {
+            (route_w == TT_ROUTE_CHUNK
+                 ? ttk_conv_gen_dw(gd, x, gw->dev, dbd, q) == 0
+                 : conv_dw_deferred(gd, NULL, x, gw, gb, q) == 0 ||
+                       tt_k_conv2d_dw_lds(gd, x, gw->dev, dbd, N, C, H, W, F, HH, WW, sh, sw, ph,
+                                          pw, Ho, Wo) == 0)) {
             if (gb) accum_move(b, gb);
             accum_move(w, gw);
             w_done = 1;
@@ -1272,11 +1275,14 @@ static void backward_conv2d(AGNode *n) {
         }
     }
     if (chained) return;
-    if (needs(a) && (lds & 4)) {
+    const int route_x = needs(a) ? ttk_conv_route(q, 2) : 0;
+    if (route_x) {
         const float *wd = tt_dev(w->val);
         Tensor *ga = wd ? tt_empty_like(a->val) : NULL;
-        if (ga && tt_k_conv2d_dx_lds(gd, wd, ga->dev, N, C, H, W, F, HH, WW, sh, sw, ph, pw, Ho,
-                                     Wo) == 0) {
+        if (ga && (route_x == TT_ROUTE_CHUNK
+                       ? ttk_conv_gen_dx(gd, wd, ga->dev, q)
+                       : tt_k_conv2d_dx_lds(gd, wd, ga->dev, N, C, H, W, F, HH, WW, sh, sw, ph,
+                                            pw, Ho, Wo)) == 0) {
             accum_move(a, ga);
             return;
         }

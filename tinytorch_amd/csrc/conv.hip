@@ -3094,3 +3094,65 @@ extern "C" int tt_k_conv2d_chain_bwd(const float *dc2, const float *w2,
   if (rc != 0) return rc;
   return ttk_dwt_reduce_jobs(job, dw2 ? 2 : 1);
 }
+
+extern "C" int ttk_fail_direct_conv(void) { return fail_direct(); }
+
+namespace {
+
+// Estimated microseconds of the input gradient: the chunked kernel multiplies
+// 32 input channels whatever C is (95 TFLOP/s measured where its grid fills
+// the chip, and a chunk's round trip of 1 us and 10 ns an index where it does
+// not); the GEMM of the column gradient wastes nothing (60 TFLOP/s) but moves
+// the C * taps * pixels matrix out and back through col2im (measured: 64 x 8 x
+// 30 x 30 -> 200: 95 against 53 us; 24 x 16 x 16 x 16 -> 100, 5 x 5: 39 against
+// 27; 404 x 16 x 16 x 16 -> 32, 5 x 5: 67 against 111; 32 x 64 x 56 x 56 -> 128:
+// 168 against 253).
+double dx_chunk_us(const Geo &g, int N) {
+  const double taps = (double)g.HH * g.WW, px = (double)N * g.Ho * g.Wo;
+  const double work = 2.0 * ((g.C + 31) / 32 * 32) * g.F * taps * px / 95e6;
+  const double serial = (g.F + 7) / 8 * (1 + 0.08 * taps / (g.sh * g.sw));
+  return (work > serial ? work : serial) + 6;
+}
+double dx_gemm_us(const Geo &g, int N) {
+  const double taps = (double)g.HH * g.WW, px = (double)N * g.Ho * g.Wo;
+  return 2.0 * g.C * g.F * taps * px / 60e6 + 8.0 * g.C * taps * px / 2.5e6 + 8;
+}
+
+}  // namespace
+
+// Which kernel a convolution of this geometry takes (what: 0 forward, 1
+// weight gradient, 2 input gradient): TT_ROUTE_SLAB the kernels here that
+// hold the rows of every channel in LDS, TT_ROUTE_CHUNK those of
+// conv_gen.hip, 0 neither (im2col + GEMM).  Where both cover a shape, the
+// slab kernels are the faster ones for 3x3 stride-1 taps with 16-byte rows
+// (128 x 32 x 16 x 16 -> 64: forward 17.7 us against 21.0, dX 16.9 / 27; with
+// 14-float rows 17.0 / 14.5 and 15.1 / 23), for few channels (128 x 3 x 32
+// x 32 -> 32: 10.2 / 17; dW of 64 x 6 x 30 x 30 -> 64: 24.7 / 38), and the
+// tiled weight gradient where its units fit (25.1 / 37; 404 x 16 x 16 x 16 ->
+// 32, 5 x 5: 60 / 68) except over many filters and taps (32 x 64 x 56 x 56 ->
+// 128: 212 / 190); elsewhere the chunked ones (50 x 24 x 45 x 37 -> 40, 5 x 5,
+// stride 2: forward 72 / 31; 404 x 16 x 16 x 16 -> 32, 5 x 5: dX 119 / 67; 41 x
+// 41 x 64 x 63 -> 26, stride 2: dW 82 / 38).
+extern "C" int ttk_conv_route(const int q[13], int what) {
+  const int N = q[0], C = q[1], H = q[2], W = q[3], F = q[4], HH = q[5], WW = q[6], sh = q[7],
+            sw = q[8], ph = q[9], pw = q[10], Ho = q[11], Wo = q[12];
+  if (!g_lds_conv || !geo_ok(N, C, H, W, F, HH, WW, sh, sw, ph, pw, Ho, Wo)) return 0;
+  const Geo g{C, H, W, HH, WW, sh, sw, ph, pw, Ho, Wo, F, C * HH * WW};
+  const bool slab = tt_k_conv2d_lds_plan(N, C, H, W, F, HH, WW, sh, sw, ph, pw, Ho, Wo) >> what & 1;
+  bool keep;   // the slab kernel where it covers the shape
+  bool chunk;  // the chunked one covers it
+  if (what == 0) {
+    keep = C < 8 || (is_k3(g) && sh == 1 && sw == 1 &&
+                     (W % 4 == 0 || (slab && pool_fusable(g, plan_fwd(g, N, false)))));
+    chunk = ttk_conv_gen_fwd(nullptr, nullptr, nullptr, nullptr, nullptr, q) == 0;
+  } else if (what == 1) {
+    keep = C < 8 || (g_dwt && plan_dwt(g, N).tg && (long)F * g.K < 65536);
+    chunk = ttk_conv_gen_dw(nullptr, nullptr, nullptr, nullptr, q) == 0;
+  } else {
+    keep = is_k3(g);
+    chunk = ttk_conv_gen_dx(nullptr, nullptr, nullptr, q) == 0;
+    if (!(slab && keep) && dx_gemm_us(g, N) < dx_chunk_us(g, N)) return 0;
+  }
+  if (slab && (keep || !chunk)) return TT_ROUTE_SLAB;
+  return chunk ? TT_ROUTE_CHUNK : 0;
+}

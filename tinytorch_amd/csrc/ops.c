@@ -248,10 +248,21 @@ static int conv_fwd_gemm(const float *x, const float *wd, const float *bd, float
     return rc ? -3 : 0;
 }
 
+/* out = conv(x, w) + b and, when rout is given, its relu, by the direct
+ * kernel that the geometry takes; 0 ok, else nothing was written. */
+static int conv_fwd_direct(const float *x, const float *w, const float *b, float *out,
+                           float *rout, const int *q) {
+    const int route = ttk_conv_route(q, 0);
+    if (route == TT_ROUTE_CHUNK) return ttk_conv_gen_fwd(x, w, b, out, rout, q);
+    if (rout)
+        return tt_k_conv2d_relu_fwd_lds(x, w, b, out, rout, q[0], q[1], q[2], q[3], q[4], q[5],
+                                        q[6], q[7], q[8], q[9], q[10], q[11], q[12]);
+    return tt_k_conv2d_fwd_lds(x, w, b, out, q[0], q[1], q[2], q[3], q[4], q[5], q[6], q[7],
+                               q[8], q[9], q[10], q[11], q[12]);
+}
+
 int tt_conv_fwd_any(const float *x, const float *w, const float *b, float *out, const int *q) {
-    if (tt_k_conv2d_fwd_lds(x, w, b, out, q[0], q[1], q[2], q[3], q[4], q[5], q[6], q[7], q[8],
-                            q[9], q[10], q[11], q[12]) == 0)
-        return 0;
+    if (conv_fwd_direct(x, w, b, out, NULL, q) == 0) return 0;
     return conv_fwd_gemm(x, w, b, out, q);
 }
 
@@ -407,9 +418,8 @@ static int flush_one(void) {
         if (rc == 0 && tt_lazy_relu(tt_pend.r, tt_pend.out) != 0)
             rc = tt_k_relu_fwd(tt_pend.out->dev, tt_pend.r->dev, tt_pend.r->numel) ? -2 : 0;
         if (rc != 0) {  /* the convolution + relu, then the pool and the copy by themselves */
-            rc = tt_k_conv2d_relu_fwd_lds(tt_pend.x, tt_pend.w, tt_pend.b, tt_pend.out->dev,
-                                          tt_pend.r->dev, q[0], q[1], q[2], q[3], q[4], q[5],
-                                          q[6], q[7], q[8], q[9], q[10], q[11], q[12]);
+            rc = conv_fwd_direct(tt_pend.x, tt_pend.w, tt_pend.b, tt_pend.out->dev,
+                                 tt_pend.r->dev, q);
             if (rc != 0) {
                 rc = conv_fwd_gemm(tt_pend.x, tt_pend.w, tt_pend.b, tt_pend.out->dev, q);
                 if (rc == 0)
@@ -433,11 +443,7 @@ static int flush_one(void) {
             if (kind == TT_PEND_CHAIN_FC) tt_pend.fco->valid = 0;
         }
     } else {
-        const int *q = tt_pend.geo;
-        rc = tt_k_conv2d_fwd_lds(tt_pend.x, tt_pend.w, tt_pend.b, tt_pend.out->dev, q[0], q[1],
-                                 q[2], q[3], q[4], q[5], q[6], q[7], q[8], q[9], q[10], q[11],
-                                 q[12]);
-        if (rc != 0) rc = conv_fwd_gemm(tt_pend.x, tt_pend.w, tt_pend.b, tt_pend.out->dev, q);
+        rc = tt_conv_fwd_any(tt_pend.x, tt_pend.w, tt_pend.b, tt_pend.out->dev, tt_pend.geo);
     }
     if (rc != 0) {
         tt_pend.out->valid = 0;
@@ -490,10 +496,9 @@ Tensor *tt_conv2d_keepcol_ex(const Tensor *a, const Tensor *w, const Tensor *b, 
     }
     const int Kc = C * HH * WW;
     const long Ncol = (long)N * Ho * Wo;
-    /* LDS-staged direct convolution: taken when it also covers the weight
+    /* direct convolution: taken when a direct kernel also covers the weight
      * gradient the caller will ask for (that reads x, so no col is kept) */
-    const int lds = tt_k_conv2d_lds_plan(N, C, H, W, F, HH, WW, sh, sw, ph, pw, Ho, Wo);
-    const int direct = (lds & 1) && (!col_out || (lds & 2));
+    const int direct = ttk_conv_route(q, 0) && (!col_out || ttk_conv_route(q, 1));
     if (direct && defer && g_conv_relu) {
         tt_flush_pending();
         tt_pend.out = out;
@@ -508,11 +513,7 @@ Tensor *tt_conv2d_keepcol_ex(const Tensor *a, const Tensor *w, const Tensor *b, 
         tt_pend = first;
         if (!(x = tt_dev((Tensor *)a))) return fail(out);
     }
-    if (direct) {
-        if (tt_k_conv2d_fwd_lds(x, wd, bd, out->dev, N, C, H, W, F, HH, WW, sh, sw, ph, pw, Ho,
-                                Wo) == 0)
-            return out;
-    }
+    if (direct && conv_fwd_direct(x, wd, bd, out->dev, NULL, q) == 0) return out;
     if (tt_conv_use_implicit(sizeof(float) * (long)Kc * Ncol) &&
         tt_k_conv2d_fwd_implicit(x, wd, bd, out->dev, N, C, H, W, F, HH, WW, sh, sw, ph, pw, Ho,
                                  Wo) == 0)

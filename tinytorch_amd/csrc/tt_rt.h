@@ -123,6 +123,22 @@ typedef struct {
 } TTTnSgdJob;
 int    ttk_gemm_tn_padones_sgd_jobs(const TTTnSgdJob *jobs, int nj, float lr, float *const *pw,
                                     const float *const *pg, const long *pn, int np);
+/* conv_gen.hip: the convolution over channel chunks, q = N C H W F HH WW sh sw
+ * ph pw Ho Wo: forward (bias, rout = its relu optional), input gradient of
+ * any stride, weight gradient (db optional).  Output NULL: only whether the
+ * shape is covered.  0 ok, -1 not covered, -2 no memory, -3 launch failed. */
+int    ttk_conv_gen_fwd(const float *x, const float *w, const float *bias, float *out,
+                        float *rout, const int q[13]);
+int    ttk_conv_gen_dx(const float *gr, const float *w, float *dx, const int q[13]);
+int    ttk_conv_gen_dw(const float *gr, const float *x, float *dw, float *db, const int q[13]);
+/* tuning: force the plans (tile, channels a chunk, dW tile, splits; -1 / 0:
+ * automatic) */
+void   ttk_conv_gen_force(int tile, int ck, int dw, int splits);
+/* conv.hip: the kernel of a convolution (what: 0 forward, 1 dW, 2 dX) */
+#define TT_ROUTE_SLAB 1
+#define TT_ROUTE_CHUNK 2
+int    ttk_conv_route(const int q[13], int what);
+int    ttk_fail_direct_conv(void);      /* TT_FAIL_DIRECT_CONV is set */
 /* conv.hip: free a job's partials without reducing them */
 void   ttk_dwt_job_drop(TTDwtJob *job);
 /* elementwise.hip: C = A * B + bias (A M x K, B K x N row-major) for N <= 16,
