@@ -1,0 +1,74 @@
+"""Softmax-CE with the rows over many workgroups, at the edges of its lane
+groups, label forms and row counts, against float64."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from tinytorch_amd.hip import DevBuf, check
+
+pytestmark = pytest.mark.gpu
+
+
+def _ref(x, y):
+    x64 = x.astype(np.float64)
+    p = np.exp(x64 - x64.max(1, keepdims=True))
+    p /= p.sum(1, keepdims=True)
+    ok = (y >= 0) & (y < x.shape[1])
+    py = np.where(ok, p[np.arange(len(y)), np.where(ok, y, 0)], 0.0)
+    seed = p.copy()
+    seed[np.arange(len(y))[ok], y[ok]] -= 1.0
+    return p, seed / len(y), -np.log(np.maximum(py, 1e-12))
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (257, 10), (256, 17), (600, 32), (513, 33), (3072, 64),
+                                       (3073, 65), (5, 128), (40, 129), (300, 255), (33, 256),
+                                       (65, 257), (9, 1000), (20000, 10)])
+def test_softmax_ce_rows(tlib, rows, cols):
+    """Every group width (16, 32, 64 lanes, a wavefront) and label form (two
+    byte arrays in the arguments, device memory); fp32 exponentials and sums
+    of `cols` terms stay within 1e-5 of float64."""
+    from tinytorch_amd.torch_py import Node
+    rng = np.random.default_rng(rows * 1000 + cols)
+    x = (rng.standard_normal((rows, cols)) * 3).astype(np.float32)
+    y = rng.integers(0, cols, rows).astype(np.int32)
+    if rows > 4:
+        y[1], y[3] = -1, cols  # labels outside: no column, the clamped loss
+    p64, s64, l64 = _ref(x, y)
+    X = Node.leaf(x)
+    loss = X.softmax_ce(y)
+    loss.backward(None)
+    np.testing.assert_allclose(loss.probs(), p64, rtol=1e-5, atol=1e-7)
+    # p_y - 1 cancels: the probability's own error, about 4 ulp of 1 (expf,
+    # the sum, the division), stays as 2.4e-7 of the seed's scale
+    np.testing.assert_allclose(X.grad(), s64, rtol=1e-5, atol=4e-7 / rows)
+    np.testing.assert_allclose(loss.value(), [l64.mean()], rtol=1e-5)
+    loss.backward(None)  # recomputed from the kept labels and added
+    np.testing.assert_allclose(X.grad(), 2 * s64, rtol=1e-5, atol=8e-7 / rows)
+    # the device entry, its mean added in the order of the row losses
+    dx, dl = DevBuf.from_np(x), DevBuf.from_np(y)
+    pr, se, me, lo = DevBuf(x.size), DevBuf(x.size), DevBuf(1), DevBuf(rows)
+    sc = ctypes.c_float(1.0 / rows)
+    check(tlib.tt_k_softmax_ce(dx.ptr, dl.ptr, pr.ptr, lo.ptr, se.ptr, rows, cols, sc), "ce")
+    np.testing.assert_allclose(lo.to_np((rows,)), l64, rtol=1e-5, atol=1e-5)
+    if rows <= 8192:
+        check(tlib.tt_k_softmax_ce_mean(dx.ptr, dl.ptr, pr.ptr, me.ptr, se.ptr, rows, cols, sc), "mean")
+        check(tlib.tt_k_ce_mean_rows(lo.ptr, lo.ptr, rows), "mean of the rows")
+        assert me.to_np((1,))[0] == lo.to_np((rows,))[0]
+    for n in (loss, X):
+        n.release()
+
+
+def test_softmax_small_rows(tlib):
+    """Rows of up to 64 columns by groups of lanes, with a row of -inf."""
+    rng = np.random.default_rng(3)
+    for rows, cols in ((1, 10), (17, 16), (5, 17), (100, 64), (3, 1)):
+        x = rng.standard_normal((rows, cols)).astype(np.float32)
+        x[rows // 2] = -np.inf
+        d, y = DevBuf.from_np(x), DevBuf(x.size)
+        check(tlib.tt_k_softmax_fwd(d.ptr, y.ptr, rows, cols), "softmax")
+        got = y.to_np(x.shape)
+        assert np.all(got[rows // 2] == np.float32(1.0) / np.float32(cols))
+        keep = np.arange(rows) != rows // 2
+        e = np.exp(x[keep].astype(np.float64) - x[keep].max(1, keepdims=True, initial=-1e30))
+        np.testing.assert_allclose(got[keep], e / e.sum(1, keepdims=True), rtol=1e-5)

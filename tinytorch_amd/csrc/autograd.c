@@ -718,56 +718,24 @@ AGNode *ag_softmax_ce(AGNode *logits, const int *labels, long rows) {
         tt_release(probs); tt_release(seed); tt_release(loss); free(hlab);
         return NULL;
     }
-    /* small batches: the labels travel inside the kernel's arguments */
-    if (probs && seed && loss && hlab && rows <= TT_CE_ARG_ROWS &&
-        tt_k_softmax_ce_mean_hostlab(x, hlab, probs->dev, loss->dev, seed->dev, rows, cols,
-                                     1.0f / (float)rows) == 0) {
-        AGNode *n = make_node(loss, &OP_SOFTMAX_CE, logits, NULL, NULL);
-        if (!n) { tt_release(probs); tt_release(seed); free(hlab); return NULL; }
-        n->at.ce.probs = probs;
-        n->at.ce.seed = seed;
-        n->at.ce.labels = hlab;
-        return n;
-    }
-    free(hlab);
-    int32_t *dlab = (int32_t *)ttrt_alloc(sizeof(int32_t) * (size_t)rows);
-    float *rowloss = rows > TT_CE_MEAN_MAX_ROWS ? (float *)ttrt_alloc(sizeof(float) * (size_t)rows)
-                                                : NULL;
-    int ok = probs && seed && loss && dlab && (rowloss || rows <= TT_CE_MEAN_MAX_ROWS);
-    if (ok) {
-        int32_t *h = (int32_t *)malloc(sizeof(int32_t) * (size_t)rows);
-        ok = h != NULL;
-        if (ok) {
-            for (long r = 0; r < rows; r++) h[r] = (int32_t)labels[r];
-            ok = ttrt_h2d_async(dlab, h, sizeof(int32_t) * (size_t)rows) == 0;
-            free(h);
-        }
-    }
-    /* small batches: one workgroup computes probabilities, seed and the mean
-     * loss; large ones reduce the per-row losses with a 1 x rows x 1 GEMM
-     * against a vector of 1/rows */
-    float *inv = NULL;
-    if (ok && rows <= TT_CE_MEAN_MAX_ROWS) {
-        ok = tt_k_softmax_ce_mean(x, dlab, probs->dev, loss->dev, seed->dev, rows, cols,
-                                  1.0f / (float)rows) == 0;
-    } else if (ok) {
-        inv = (float *)ttrt_alloc(sizeof(float) * (size_t)rows);
-        ok = inv && tt_k_fill(inv, rows, 1.0f / (float)rows) == 0 &&
-             tt_k_softmax_ce(x, dlab, probs->dev, rowloss, seed->dev, rows, cols,
-                             1.0f / (float)rows) == 0 &&
-             tt_k_gemm(1, 1, (int)rows, rowloss, (int)rows, 0, inv, 1, 0, loss->dev, 1) == 0;
-    }
-    ttrt_free(dlab);
-    ttrt_free(rowloss);
-    ttrt_free(inv);
+    /* the rows' softmax-CE in one launch; the mean loss a recipe of the row
+     * losses, as above */
+    Tensor *rl = tt_empty_dev(&rows, 1);
+    const int ok = probs && seed && loss && hlab && rl &&
+                   ttk_ce_rows(x, hlab, probs->dev, seed->dev, rl->dev, rows, cols,
+                               1.0f / (float)rows) == 0 &&
+                   (tt_lazy_ce_mean(loss, rl) == 0 ||
+                    tt_k_ce_mean_rows(rl->dev, loss->dev, (int)rows) == 0);
+    tt_release(rl);
     if (!ok) {
-        tt_release(probs); tt_release(seed); tt_release(loss);
+        tt_release(probs); tt_release(seed); tt_release(loss); free(hlab);
         return NULL;
     }
     AGNode *n = make_node(loss, &OP_SOFTMAX_CE, logits, NULL, NULL);
-    if (!n) { tt_release(probs); tt_release(seed); return NULL; }
+    if (!n) { tt_release(probs); tt_release(seed); free(hlab); return NULL; }
     n->at.ce.probs = probs;
     n->at.ce.seed = seed;
+    n->at.ce.labels = hlab;
     return n;
 }
 
@@ -1458,12 +1426,10 @@ static void backward_softmax_ce(AGNode *n) {
         const long rows = a->val->shape[0];
         const int cols = (int)a->val->shape[1];
         Tensor *p = tt_empty_like(a->val), *s = tt_empty_like(a->val);
-        float *l = (float *)ttrt_alloc(sizeof(float));
-        const int ok = x && p && s && l &&
-                       tt_k_softmax_ce_mean_hostlab(x, n->at.ce.labels, p->dev, l, s->dev, rows, cols,
-                                                    1.0f / (float)rows) == 0;
+        const int ok = x && p && s &&
+                       ttk_ce_rows(x, n->at.ce.labels, p->dev, s->dev, NULL, rows, cols,
+                                   1.0f / (float)rows) == 0;
         tt_release(p);
-        ttrt_free(l);
         if (!ok) { tt_release(s); return; }
         n->at.ce.seed = s;
     }

@@ -12,17 +12,20 @@
 // before the launch), one byte each: a label outside [0, cols) is stored as
 // 255, which is outside [0, cols) too for cols <= 255 -- the same loss and
 // seed as the original label.
-struct LabU8 {
-  uint8_t v[TT_CE_ARG_ROWS];
+template <int ROWS>
+struct LabBytes {
+  uint8_t v[ROWS];
   __device__ int operator[](int r) const { return v[r]; }
 };
+using LabU8 = LabBytes<TT_CE_ARG_ROWS>;
 
-static inline void lab_u8_fill(LabU8 &la, const int32_t *host_labels, long rows, int cols) {
+template <int ROWS>
+static inline void lab_u8_fill(LabBytes<ROWS> &la, const int32_t *host_labels, long rows, int cols) {
   for (long r = 0; r < rows; r++) {
     const int32_t y = host_labels[r];
     la.v[r] = (uint8_t)(y >= 0 && y < cols ? y : 255);
   }
-  for (long r = rows; r < TT_CE_ARG_ROWS; r++) la.v[r] = 255;
+  for (long r = rows; r < ROWS; r++) la.v[r] = 255;
 }
 
 // Probabilities and seed (p - onehot(y)) * scale of one row of cols logits
@@ -89,6 +92,7 @@ __device__ __forceinline__ void ce_rows_block(const float *__restrict__ x, const
   ce_mean_tree(acc, part, loss_mean, rows);
 }
 
+// softmax_row_group: the probabilities of a row by a group of lanes; ce_row_group:
 // ce_row by a group of W lanes (W a power of two, the group's lanes
 // consecutive and all active), CPL columns a lane (cols <= W * CPL): lane q =
 // threadIdx.x % W holds the logits of columns q * CPL + u in x[u] (ignored
@@ -99,8 +103,8 @@ __device__ __forceinline__ void ce_rows_block(const float *__restrict__ x, const
 // exponentials in column order (each lane adds the group's values one by one
 // from 0), one division a column.
 template <int W, int CPL>
-__device__ __forceinline__ float ce_row_group(const float (&x)[CPL], int y, int cols, float scale,
-                                              float (&pj)[CPL], float (&sj)[CPL]) {
+__device__ __forceinline__ void softmax_row_group(const float (&x)[CPL], int cols,
+                                                  float (&v)[CPL]) {
   const int q = threadIdx.x & (W - 1);
   float mx = -INFINITY;
 #pragma unroll
@@ -111,7 +115,6 @@ __device__ __forceinline__ float ce_row_group(const float (&x)[CPL], int y, int 
     const float t = __shfl_xor(mx, o, W);
     if (t > mx) mx = t;
   }
-  float v[CPL];
   if (mx == -INFINITY) {
 #pragma unroll
     for (int u = 0; u < CPL; u++) v[u] = 1.0f / (float)cols;
@@ -128,13 +131,19 @@ __device__ __forceinline__ float ce_row_group(const float (&x)[CPL], int y, int 
 #pragma unroll
     for (int u = 0; u < CPL; u++) v[u] = e[u] / sum;
   }
+}
+
+template <int W, int CPL>
+__device__ __forceinline__ float ce_row_group(const float (&x)[CPL], int y, int cols, float scale,
+                                              float (&pj)[CPL], float (&sj)[CPL]) {
+  const int q = threadIdx.x & (W - 1);
+  softmax_row_group<W, CPL>(x, cols, pj);
   float py = 0.0f;
 #pragma unroll
   for (int u = 0; u < CPL; u++) {
     const int j = q * CPL + u;
-    pj[u] = v[u];
-    sj[u] = (v[u] - (j == y ? 1.0f : 0.0f)) * scale;
-    if (j == y) py = v[u];
+    sj[u] = (pj[u] - (j == y ? 1.0f : 0.0f)) * scale;
+    if (j == y) py = pj[u];
   }
   // the lane that holds column y has its probability, the others 0 (and all
   // 0 for a label out of range): the largest over the group is p_y

@@ -132,23 +132,22 @@ struct SgdOp {
 // sequential summation order; wider rows run one row per wavefront with a
 // butterfly reduction.
 
-// softmax, one row per thread (cols <= 64)
-__global__ void softmax_rowthread_kernel(const float *__restrict__ x, float *__restrict__ y,
-                                         long rows, int cols) {
-  const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// softmax, W lanes a row, CPL columns a lane (cols <= W * CPL): the bits of
+// one thread a row summing the columns in order (softmax_row_group), without
+// its serial loads -- one row of 10 took 4.3 us by one thread, 1.9 by 16 lanes.
+template <int W, int CPL>
+__global__ void __launch_bounds__(256)
+softmax_group_kernel(const float *__restrict__ x, float *__restrict__ y, long rows, int cols) {
+  const long r = (long)blockIdx.x * (256 / W) + threadIdx.x / W;
+  const int q = threadIdx.x & (W - 1);
   if (r >= rows) return;
-  const float *xr = x + r * cols;
-  float *yr = y + r * cols;
-  float mx = -INFINITY;
-  for (int j = 0; j < cols; j++) { const float v = xr[j]; if (v > mx) mx = v; }
-  if (mx == -INFINITY) {
-    const float u = 1.0f / (float)cols;
-    for (int j = 0; j < cols; j++) yr[j] = u;
-    return;
-  }
-  float sum = 0.0f;
-  for (int j = 0; j < cols; j++) { const float e = expf(xr[j] - mx); yr[j] = e; sum += e; }
-  for (int j = 0; j < cols; j++) yr[j] = yr[j] / sum;
+  float v[CPL], p[CPL];
+#pragma unroll
+  for (int u = 0; u < CPL; u++) v[u] = q * CPL + u < cols ? x[r * cols + q * CPL + u] : 0.0f;
+  softmax_row_group<W, CPL>(v, cols, p);
+#pragma unroll
+  for (int u = 0; u < CPL; u++)
+    if (q * CPL + u < cols) y[r * cols + q * CPL + u] = p[u];
 }
 
 __device__ __forceinline__ float wave_max(float v) {
@@ -205,28 +204,73 @@ __global__ void softmax_bwd_rowwave_kernel(const float *__restrict__ s, const fl
 }
 
 // Fused softmax + cross-entropy: probs, per-row loss -log(max(p[y],1e-12))
-// and the logits gradient seed (p - onehot(y)) * scale, one row per thread.
-__global__ void softmax_ce_kernel(const float *__restrict__ x, const int32_t *__restrict__ lab,
-                                  float *__restrict__ probs, float *__restrict__ loss,
-                                  float *__restrict__ seed, long rows, int cols, float scale) {
-  const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// and the logits gradient seed (p - onehot(y)) * scale, by W lanes a row
+// (ce_row_group, cols <= W * CPL), the rows over as many workgroups as they
+// fill.  LAB: a device pointer to the labels or the labels themselves.
+template <int W, int CPL, class LAB>
+__global__ void __launch_bounds__(256)
+softmax_ce_group_kernel(const float *__restrict__ x, const LAB lab, float *__restrict__ probs,
+                        float *__restrict__ loss, float *__restrict__ seed, int rows, int cols,
+                        float scale) {
+  const int r = blockIdx.x * (256 / W) + threadIdx.x / W;
+  const int q = threadIdx.x & (W - 1);
   if (r >= rows) return;
-  const float *xr = x + r * cols;
-  float *pr = probs + r * cols;
-  float mx = -INFINITY;
-  for (int j = 0; j < cols; j++) { const float v = xr[j]; if (v > mx) mx = v; }
-  if (mx == -INFINITY) {
-    for (int j = 0; j < cols; j++) pr[j] = 1.0f / (float)cols;
-  } else {
-    float sum = 0.0f;
-    for (int j = 0; j < cols; j++) { const float e = expf(xr[j] - mx); pr[j] = e; sum += e; }
-    for (int j = 0; j < cols; j++) pr[j] = pr[j] / sum;
-  }
+  const long o = (long)r * cols;
+  float v[CPL], p[CPL], s[CPL];
+#pragma unroll
+  for (int u = 0; u < CPL; u++) v[u] = q * CPL + u < cols ? x[o + q * CPL + u] : 0.0f;
+  const float l = ce_row_group<W, CPL>(v, lab[r], cols, scale, p, s);
+#pragma unroll
+  for (int u = 0; u < CPL; u++)
+    if (q * CPL + u < cols) {
+      probs[o + q * CPL + u] = p[u];
+      seed[o + q * CPL + u] = s[u];
+    }
+  if (q == 0 && loss) loss[r] = l;
+}
+
+// the same for any number of columns, a wavefront a row
+template <class LAB>
+__global__ void __launch_bounds__(256)
+softmax_ce_wave_kernel(const float *__restrict__ x, const LAB lab, float *__restrict__ probs,
+                       float *__restrict__ loss, float *__restrict__ seed, int rows, int cols,
+                       float scale) {
+  const int r = blockIdx.x * 4 + threadIdx.x / 64;
+  const int lane = threadIdx.x & 63;
+  if (r >= rows) return;
+  const float *xr = x + (long)r * cols;
+  float *pr = probs + (long)r * cols, *sr = seed + (long)r * cols;
   const int y = lab[r];
-  const bool ok = y >= 0 && y < cols;
-  const float py = ok ? pr[y] : 0.0f;
-  loss[r] = -logf(fmaxf(py, 1e-12f));
-  for (int j = 0; j < cols; j++) seed[r * cols + j] = (pr[j] - (j == y ? 1.0f : 0.0f)) * scale;
+  float mx = -INFINITY;
+  for (int j = lane; j < cols; j += 64) { const float v = xr[j]; if (v > mx) mx = v; }
+  mx = wave_max(mx);
+  float sum = 0.0f;
+  if (mx != -INFINITY)
+    for (int j = lane; j < cols; j += 64) sum += expf(xr[j] - mx);
+  sum = wave_sum(sum);
+  float py = 0.0f;
+  for (int j = lane; j < cols; j += 64) {
+    const float p = mx == -INFINITY ? 1.0f / (float)cols : expf(xr[j] - mx) / sum;
+    pr[j] = p;
+    sr[j] = (p - (j == y ? 1.0f : 0.0f)) * scale;
+    if (j == y) py = p;
+  }
+  for (int k = 32; k > 0; k >>= 1) py = fmaxf(py, __shfl_xor(py, k, 64));
+  if (lane == 0 && loss) loss[r] = -logf(fmaxf(py, 1e-12f));
+}
+
+// the mean loss from the probabilities, added as ce_rows_block adds its rows'
+template <class LAB>
+__global__ void __launch_bounds__(256)
+ce_mean_probs_kernel(const float *__restrict__ probs, const LAB lab, float *__restrict__ loss_mean,
+                     int rows, int cols) {
+  __shared__ float part[256];
+  float acc = 0.0f;
+  for (int r = threadIdx.x; r < rows; r += 256) {
+    const int y = lab[r];
+    acc += -logf(fmaxf(y >= 0 && y < cols ? probs[(long)r * cols + y] : 0.0f, 1e-12f));
+  }
+  ce_mean_tree(acc, part, loss_mean, rows);
 }
 
 template <typename I>
@@ -354,41 +398,6 @@ softmax_ce_mean_kernel(const float *__restrict__ x, const LAB lab, float *__rest
                        int cols, float scale) {
   __shared__ float part[256];
   ce_rows_block<MAXC>(x, lab, probs, loss_mean, seed, rows, cols, scale, part);
-}
-
-// general width: the same passes over global memory
-template <class LAB>
-__global__ void softmax_ce_mean_wide_kernel(const float *__restrict__ x, const LAB lab,
-                                            float *__restrict__ probs,
-                                            float *__restrict__ loss_mean,
-                                            float *__restrict__ seed, int rows, int cols,
-                                            float scale) {
-  __shared__ float part[256];
-  float acc = 0.0f;
-  for (int r = threadIdx.x; r < rows; r += blockDim.x) {
-    const float *xr = x + (long)r * cols;
-    float *pr = probs + (long)r * cols;
-    float mx = -INFINITY;
-    for (int j = 0; j < cols; j++) { const float v = xr[j]; if (v > mx) mx = v; }
-    if (mx == -INFINITY) {
-      for (int j = 0; j < cols; j++) pr[j] = 1.0f / (float)cols;
-    } else {
-      float sum = 0.0f;
-      for (int j = 0; j < cols; j++) { const float e = expf(xr[j] - mx); pr[j] = e; sum += e; }
-      for (int j = 0; j < cols; j++) pr[j] = pr[j] / sum;
-    }
-    const int y = lab[r];
-    const float py = (y >= 0 && y < cols) ? pr[y] : 0.0f;
-    acc += -logf(fmaxf(py, 1e-12f));
-    for (int j = 0; j < cols; j++) seed[(long)r * cols + j] = (pr[j] - (j == y ? 1.0f : 0.0f)) * scale;
-  }
-  part[threadIdx.x] = acc;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) part[threadIdx.x] += part[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) loss_mean[0] = part[0] / (float)rows;
 }
 
 // y = x * s[0] with s a device scalar (the incoming gradient of a scalar loss)
@@ -896,9 +905,12 @@ int tt_k_sgd(float *w, const float *g, long n, float lr) {
 
 int tt_k_softmax_fwd(const float *x, float *y, long rows, int cols) {
   if (rows <= 0 || cols <= 0) return 0;
-  if (cols <= 64) {
-    hipLaunchKernelGGL(softmax_rowthread_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0,
-                       stream(), x, y, rows, cols);
+  if (cols <= 16 && rows <= 0x7fffffffL) {
+    hipLaunchKernelGGL((softmax_group_kernel<16, 1>), dim3((unsigned)((rows + 15) / 16)), dim3(256),
+                       0, stream(), x, y, rows, cols);
+  } else if (cols <= 64 && rows <= 0x7fffffffL) {
+    hipLaunchKernelGGL((softmax_group_kernel<16, 4>), dim3((unsigned)((rows + 15) / 16)), dim3(256),
+                       0, stream(), x, y, rows, cols);
   } else {
     hipLaunchKernelGGL(softmax_rowwave_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0,
                        stream(), x, y, rows, cols);
@@ -918,12 +930,56 @@ int tt_k_softmax_bwd(const float *s, const float *g, float *dx, long rows, int c
   return launched();
 }
 
+extern "C++" template <class LAB>
+static void launch_ce_rows(const float *x, const LAB &lab, float *probs, float *loss, float *seed,
+                           int rows, int cols, float scale) {
+#define TT_CE(W_, CPL_)                                                                       \
+  hipLaunchKernelGGL((softmax_ce_group_kernel<W_, CPL_, LAB>),                                \
+                     dim3((unsigned)((rows + 256 / W_ - 1) / (256 / W_))), dim3(256), 0,      \
+                     stream(), x, lab, probs, loss, seed, rows, cols, scale)
+  if (cols <= 16) TT_CE(16, 1);
+  else if (cols <= 32) TT_CE(16, 2);
+  else if (cols <= 64) TT_CE(16, 4);
+  else if (cols <= 128) TT_CE(32, 4);
+  else if (cols <= 256) TT_CE(64, 4);
+  else
+    hipLaunchKernelGGL((softmax_ce_wave_kernel<LAB>), dim3((unsigned)((rows + 3) / 4)), dim3(256),
+                       0, stream(), x, lab, probs, loss, seed, rows, cols, scale);
+#undef TT_CE
+}
+
 int tt_k_softmax_ce(const float *logits, const int32_t *labels, float *probs, float *loss_rows,
                     float *seed, long rows, int cols, float scale) {
   if (rows <= 0 || cols <= 0) return 0;
-  hipLaunchKernelGGL(softmax_ce_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, stream(),
-                     logits, labels, probs, loss_rows, seed, rows, cols, scale);
+  if (rows > 0x7fffffffL) return -1;
+  launch_ce_rows(logits, labels, probs, loss_rows, seed, (int)rows, cols, scale);
   return launched();
+}
+
+int ttk_ce_rows(const float *logits, const int32_t *host_labels, float *probs, float *seed,
+                float *rowloss, long rows, int cols, float scale) {
+  if (rows <= 0 || cols <= 0 || rows > 0x7fffffffL || !host_labels) return -1;
+  constexpr int BIG = 3072;
+  if (cols <= 255 && rows <= TT_CE_ARG_ROWS) {
+    LabU8 la;
+    lab_u8_fill(la, host_labels, rows, cols);
+    launch_ce_rows(logits, la, probs, rowloss, seed, (int)rows, cols, scale);
+    return launched();
+  }
+  if (cols <= 255 && rows <= BIG) {
+    LabBytes<BIG> la;
+    lab_u8_fill(la, host_labels, rows, cols);
+    launch_ce_rows(logits, la, probs, rowloss, seed, (int)rows, cols, scale);
+    return launched();
+  }
+  int32_t *dl = (int32_t *)ttrt_alloc(sizeof(int32_t) * (size_t)rows);
+  int rc = dl && ttrt_h2d_async(dl, host_labels, sizeof(int32_t) * (size_t)rows) == 0 ? 0 : -2;
+  if (rc == 0) {
+    launch_ce_rows(logits, (const int32_t *)dl, probs, rowloss, seed, (int)rows, cols, scale);
+    rc = launched();
+  }
+  ttrt_free(dl);  // stream-ordered
+  return rc;
 }
 
 int tt_k_copy_padones_fwd(const float *x, float *c, float *y, long M, long K) {
@@ -991,15 +1047,20 @@ int tt_k_padones_bwd(const float *g, float *dx, long M, long K) {
 extern "C++" template <class LAB>
 static void launch_ce_mean(const float *logits, const LAB &labels, float *probs, float *loss_mean,
                            float *seed, long rows, int cols, float scale) {
-  if (cols <= 16)
+  // one workgroup, a row a thread, while that is one round of short rows;
+  // else the rows over many workgroups and then the mean (937 rows of 91: 417
+  // us by one workgroup)
+  if (rows <= 256 && cols <= 16) {
     hipLaunchKernelGGL((softmax_ce_mean_kernel<16, LAB>), dim3(1), dim3(256), 0, stream(), logits,
                        labels, probs, loss_mean, seed, (int)rows, cols, scale);
-  else if (cols <= 32)
+  } else if (rows <= 256 && cols <= 32) {
     hipLaunchKernelGGL((softmax_ce_mean_kernel<32, LAB>), dim3(1), dim3(256), 0, stream(), logits,
                        labels, probs, loss_mean, seed, (int)rows, cols, scale);
-  else
-    hipLaunchKernelGGL((softmax_ce_mean_wide_kernel<LAB>), dim3(1), dim3(256), 0, stream(), logits,
-                       labels, probs, loss_mean, seed, (int)rows, cols, scale);
+  } else {
+    launch_ce_rows(logits, labels, probs, (float *)nullptr, seed, (int)rows, cols, scale);
+    hipLaunchKernelGGL((ce_mean_probs_kernel<LAB>), dim3(1), dim3(256), 0, stream(), probs, labels,
+                       loss_mean, (int)rows, cols);
+  }
 }
 
 // c[m][n] += bias[n]; r = relu(c), p = [r, 1] when given (a row per

@@ -56,6 +56,11 @@ typedef struct {
     float scale;
 } TTCeHook;
 int    ttk_reduce_ce(const float *ws, float *C, int M, int N, int S, int zl, const TTCeHook *h);
+/* elementwise.hip: softmax-CE of the rows of logits, labels on the host (any
+ * number): probabilities, seed = (p - onehot) * scale and the row losses,
+ * whose mean tt_k_ce_mean_rows gives.  0 ok, -2 no memory. */
+int    ttk_ce_rows(const float *logits, const int32_t *host_labels, float *probs, float *seed,
+                   float *rowloss, long rows, int cols, float scale);
 /* head.hip: tt_k_head_bwd / tt_k_head_bwd_pool (codes non-NULL) whose
  * output gradient is the seed of a softmax-CE of the logits formed by the
  * kernel itself from two partial sums per logit (part: 2 x M x N), the bias
@@ -164,5 +169,31 @@ int    ttg_scratch_setup(void);
 
 #ifdef __cplusplus
 }
+
+#include <string.h>
+/* Plans of the geometries met last, by geometry (q, and a tag for the rest of
+ * what a plan depends on): planning a convolution takes the host 0.5-1 us, and
+ * a step asks several times for each of its layers.  Direct-mapped, 64
+ * entries; single-threaded like the library. */
+template <class PLAN>
+struct TTPlanCache {
+  struct Entry {
+    int q[13], tag, used;
+    PLAN plan;
+  } e[64];
+  template <class MAKE>
+  const PLAN &get(const int *q, int tag, MAKE make) {
+    unsigned h = (unsigned)tag;
+    for (int i = 0; i < 13; i++) h = h * 31u + (unsigned)q[i];
+    Entry &x = e[(h ^ h >> 6 ^ h >> 12) & 63];
+    if (!x.used || x.tag != tag || memcmp(x.q, q, sizeof(x.q)) != 0) {
+      x.plan = make();
+      memcpy(x.q, q, sizeof(x.q));
+      x.tag = tag;
+      x.used = 1;
+    }
+    return x.plan;
+  }
+};
 #endif
 #endif
