@@ -3115,7 +3115,15 @@ double dx_chunk_us(const Geo &g, int N) {
 }
 double dx_gemm_us(const Geo &g, int N) {
   const double taps = (double)g.HH * g.WW, px = (double)N * g.Ho * g.Wo;
-  return 2.0 * g.C * g.F * taps * px / 60e6 + 8.0 * g.C * taps * px / 2.5e6 + 8;
+  return 2.0 * g.C * g.F * taps * px / 60e6 + 8.0 * g.C * taps * px / 2.5e6 + 12;
+}
+// (the slab kernel, TFLOP/s of padded channels: 60 with 3x3 taps, 64 x 4 x 30 x
+// 30 -> 64 41 us against the GEMM's 23; else 45, 404 x 16 x 16 x 16 -> 32, 5 x
+// 5: 119 us)
+double dx_slab_us(const Geo &g, int N) {
+  const double taps = (double)g.HH * g.WW, px = (double)N * g.Ho * g.Wo;
+  const double work = 2.0 * ((g.C + 31) / 32 * 32) * g.F * taps * px;
+  return is_k3(g) ? work / 60e6 + 4 : work / 45e6 + 8;
 }
 
 }  // namespace
@@ -3133,7 +3141,9 @@ double dx_gemm_us(const Geo &g, int N) {
 // 128: 212 / 190); elsewhere the chunked ones (50 x 24 x 45 x 37 -> 40, 5 x 5,
 // stride 2: forward 72 / 31; 404 x 16 x 16 x 16 -> 32, 5 x 5: dX 119 / 67; 41 x
 // 41 x 64 x 63 -> 26, stride 2: dW 82 / 38).
-extern "C" int ttk_conv_route(const int q[13], int what) {
+namespace {
+
+int conv_route(const int q[13], int what) {
   const int N = q[0], C = q[1], H = q[2], W = q[3], F = q[4], HH = q[5], WW = q[6], sh = q[7],
             sw = q[8], ph = q[9], pw = q[10], Ho = q[11], Wo = q[12];
   if (!g_lds_conv || !geo_ok(N, C, H, W, F, HH, WW, sh, sw, ph, pw, Ho, Wo)) return 0;
@@ -3149,10 +3159,25 @@ extern "C" int ttk_conv_route(const int q[13], int what) {
     keep = C < 8 || (g_dwt && plan_dwt(g, N).tg && (long)F * g.K < 65536);
     chunk = ttk_conv_gen_dw(nullptr, nullptr, nullptr, nullptr, q) == 0;
   } else {
-    keep = is_k3(g);
     chunk = ttk_conv_gen_dx(nullptr, nullptr, nullptr, q) == 0;
-    if (!(slab && keep) && dx_gemm_us(g, N) < dx_chunk_us(g, N)) return 0;
+    const double never = 1e30, tc = chunk ? dx_chunk_us(g, N) : never, tg = dx_gemm_us(g, N),
+                 ts = slab ? dx_slab_us(g, N) : never;
+    keep = slab && (is_k3(g) || ts <= tc);  // 3x3: faster than the chunked one, above
+    if (tg < (keep ? ts : tc)) return 0;
   }
   if (slab && (keep || !chunk)) return TT_ROUTE_SLAB;
   return chunk ? TT_ROUTE_CHUNK : 0;
+}
+
+struct ConvRoute {
+  int r;
+};
+TTPlanCache<ConvRoute> g_routes;
+
+}  // namespace
+
+extern "C" int ttk_conv_route(const int q[13], int what) {
+  return g_routes
+      .get(q, what + 3 * (g_lds_conv + 2 * g_dwt), [&] { return ConvRoute{conv_route(q, what)}; })
+      .r;
 }

@@ -866,10 +866,19 @@ int launch_gen(const ConvG &g, const GenPlan &p, bool va) {
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
+struct DwPlan {
+  int tile = -1, nch = 0, per = 0, splits = 0;
+  long lds = 0, cs = 0, ftiles = 0, ctiles = 0;
+};
+TTPlanCache<GenPlan> g_gen_plans;  // tag: dX, 16-byte weights, the forced plans
+TTPlanCache<DwPlan> g_dw_plans;
+int g_force_tag = 0;
+
 template <bool DX>
-int run_gen(ConvG g, bool dry) {
+int run_gen(ConvG g, const int q[13], bool dry) {
   const bool va = !DX && (g.C * g.HH * g.WW) % 4 == 0 && (dry || aligned16(g.w));
-  const GenPlan p = plan_gen(g, DX, va);
+  const GenPlan &p = g_gen_plans.get(q, 4 * g_force_tag + 2 * DX + va,
+                                     [&] { return plan_gen(g, DX, va); });
   if (p.tile < 0 || p.ftiles * p.ptiles >= 0x7fffffffL) return -1;
   if (dry) return 0;
   if (ttk_fail_direct_conv()) return -3;
@@ -903,10 +912,6 @@ struct DwTile {
 constexpr int NDW = 3;
 constexpr DwTile DWTILES[NDW] = {{32, 128}, {64, 64}, {128, 64}};
 
-struct DwPlan {
-  int tile = -1, nch = 0, per = 0, splits = 0;
-  long lds = 0, cs = 0, ftiles = 0, ctiles = 0;
-};
 int g_force_dw = -1, g_force_splits = 0;
 
 // The tile whose filters fit F (128 of them only where the pixels still give
@@ -979,6 +984,7 @@ ConvG gen_args(const int q[13], bool dx) {
 extern "C" void ttk_conv_gen_force(int tile, int ck, int dw, int splits) {
   g_force_tile = tile;
   g_force_ck = ck;
+  g_force_tag++;  // no plan of the cache is for these
   g_force_dw = dw;
   g_force_splits = splits;
 }
@@ -988,14 +994,14 @@ extern "C" int ttk_conv_gen_fwd(const float *x, const float *w, const float *bia
   if (!geo_ok(q)) return -1;
   ConvG g = gen_args(q, false);
   g.x = x; g.w = w; g.bias = bias; g.out = out; g.rout = rout;
-  return run_gen<false>(g, !out);
+  return run_gen<false>(g, q, !out);
 }
 
 extern "C" int ttk_conv_gen_dx(const float *gr, const float *w, float *dx, const int q[13]) {
   if (!geo_ok(q)) return -1;
   ConvG g = gen_args(q, true);
   g.x = gr; g.w = w; g.out = dx;
-  return run_gen<true>(g, !dx);
+  return run_gen<true>(g, q, !dx);
 }
 
 extern "C" int ttk_conv_gen_dw(const float *gr, const float *x, float *dw, float *db,
@@ -1005,7 +1011,7 @@ extern "C" int ttk_conv_gen_dw(const float *gr, const float *x, float *dw, float
   g.g = gr; g.x = x;
   g.N = q[0]; g.C = q[1]; g.H = q[2]; g.W = q[3]; g.F = q[4]; g.HH = q[5]; g.WW = q[6];
   g.sh = q[7]; g.sw = q[8]; g.ph = q[9]; g.pw = q[10]; g.OH = q[11]; g.OW = q[12];
-  const DwPlan p = plan_dw(g);
+  const DwPlan &p = g_dw_plans.get(q, g_force_tag, [&] { return plan_dw(g); });
   if (p.tile < 0 || p.ftiles * p.ctiles * p.splits >= 0x7fffffffL) return -1;
   const int K = g.C * g.HH * g.WW;
   const long n = (long)g.F * (K + 1);
