@@ -34,6 +34,7 @@
 //     split writes a partial tile to a workspace and a second kernel sums the
 //     splits in a fixed order (deterministic, no atomics).
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 #include <stdlib.h>
 #include "tt_rt.h"
@@ -988,7 +989,7 @@ struct MidOperand {
   // R+15 of one chunk) touches every bank once (8-k rows: rows 8 apart would
   // share banks, so their two chunks swap)
   __device__ __forceinline__ static int swz(int R) {
-    return BK == 8 ? (R >> 3) & 1 : BK == 32 ? (R >> 1) & 7 : R & 15;
+    return BK == 8 ? (R >> 3) & 1 : BK == 16 ? (R >> 1) & 3 : BK == 32 ? (R >> 1) & 7 : R & 15;
   }
   unsigned voff[NL];
   const float *p;
@@ -1093,8 +1094,11 @@ struct MidOperand {
 // so no wave reads what another loaded and the K loop has no barrier (each
 // wave waits only for its own loads); the same products summed in the same
 // order as the shared ring.
+//
+// COLS: columns of B per tile (64 or 128): wave w owns 64x64 block w / NWK of
+// the tile's ROWS / 64 x COLS / 64.
 template <bool A_KC, bool B_NC, int BK, int S, int NW, int ROWS = M_T, int NWK = NW,
-          bool DW = false, bool PRIV = false>
+          bool DW = false, bool PRIV = false, int COLS = M_T>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4, 2)))
 gemm_mid_kernel(int M, int N, int K, const float *__restrict__ A, long lda,
                 const float *__restrict__ B, long ldb, float *__restrict__ C, long ldc,
@@ -1102,11 +1106,14 @@ gemm_mid_kernel(int M, int N, int K, const float *__restrict__ A, long lda,
   TT_PROBE(0, 0);
   static_assert(S >= 3, "the pipeline needs three stages");
   constexpr int NTH = 64 * NW;
-  static_assert(ROWS % M_T == 0 && NW == (ROWS / M_T) * NWK, "waves = row blocks x k slices");
-  static_assert(!PRIV || (ROWS == M_T && NWK == NW && BK == 8 * NW), "private slices: 8 k a wave");
+  constexpr int CB = COLS / M_T;  // column blocks
+  static_assert(ROWS % M_T == 0 && COLS % M_T == 0 && NW == (ROWS / M_T) * CB * NWK,
+                "waves = blocks x k slices");
+  static_assert(!PRIV || (ROWS == M_T && CB == 1 && NWK == NW && BK == 8 * NW),
+                "private slices: 8 k a wave");
   // a private ring holds one wave's operands: tiles of 8 k, loaded by that wave alone
   constexpr int OBK = PRIV ? 8 : BK, OW = PRIV ? 1 : NW, OKS = PRIV ? 1 : NWK;
-  constexpr int OPA = ROWS * OBK, OPB = M_T * OBK;  // floats per operand per stage
+  constexpr int OPA = ROWS * OBK, OPB = COLS * OBK;  // floats per operand per stage
   constexpr int STAGE = OPA + OPB;
   constexpr int PIPE = S * STAGE * (PRIV ? NW : 1), RED = NW * M_T * M_T;
   static_assert(!PRIV || S * STAGE == M_T * M_T, "a wave's sums fill its own ring");
@@ -1114,26 +1121,30 @@ gemm_mid_kernel(int M, int N, int K, const float *__restrict__ A, long lda,
   static_assert(KSUB >= 1, "tile too shallow for the waves");
   __shared__ __attribute__((aligned(16))) float smem[PIPE > RED ? PIPE : RED];
   using OA = MidOperand<A_KC, OBK, OW, ROWS, OKS, DW>;
-  using OB = MidOperand<!B_NC, OBK, OW, M_T, OKS, DW>;
+  using OB = MidOperand<!B_NC, OBK, OW, COLS, OKS, DW>;
   constexpr int NL = OA::NL + OB::NL;  // loads per wave per tile
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31;
   const int g = lane >> 5;
-  const int rb = wave / NWK, ks = wave % NWK;  // row block, k slice
+  const int rb = wave / (CB * NWK), cb = wave / NWK % CB, ks = wave % NWK;  // block, k slice
 
-  const int tiles_m = (M + ROWS - 1) / ROWS, tiles_n = (N + M_T - 1) / M_T;
+  const int tiles_m = (M + ROWS - 1) / ROWS, tiles_n = (N + COLS - 1) / COLS;
   const int ntiles = tiles_m * tiles_n;
   int pid = blockIdx.x;
-  if ((ntiles & 7) == 0) pid = (pid & 7) * (ntiles >> 3) + (pid >> 3);
+  {
+    // neighbouring tiles on one XCD: the first ntiles % 8 XCDs take one more
+    const int q = ntiles >> 3, xcd = pid & 7;
+    pid = xcd * q + min(xcd, ntiles & 7) + (pid >> 3);
+  }
   const int group = GROUP_M * tiles_n;
   const int first_m = (pid / group) * GROUP_M;
   const int gsz = min(tiles_m - first_m, GROUP_M);
   const int tm = first_m + (pid % group) % gsz;
   const int tn = (pid % group) / gsz;
   const long m0 = (long)tm * ROWS;
-  const long n0 = (long)tn * M_T;
+  const long n0 = (long)tn * COLS;
   const int kbeg = blockIdx.z * kchunk;
   const int kend = min(K, kbeg + kchunk);
   const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
@@ -1188,7 +1199,7 @@ gemm_mid_kernel(int M, int N, int K, const float *__restrict__ A, long lda,
 #pragma unroll
     for (int h = 0; h < KSUB; h++) {
       OA::frag(st, fks, rb * M_T, h, l32, g, a[h]);
-      OB::frag(st + OPA, fks, 0, h, l32, g, b[h]);
+      OB::frag(st + OPA, fks, cb * M_T, h, l32, g, b[h]);
     }
   };
   auto mfma4 = [&](float (*ca)[2][4], float (*cb)[2][4], int h, int s) {
@@ -1289,13 +1300,13 @@ gemm_mid_kernel(int M, int N, int K, const float *__restrict__ A, long lda,
   __syncthreads();
   TT_PROBE(0, 4);
 #pragma unroll
-  for (int f0 = 0; f0 < ROWS * M_T / 4; f0 += NTH) {
-    const int f = f0 + tid;  // float4 index: row f / 16, columns 4 * (f % 16) ..
-    const int mr = f >> 4, n = 4 * (f & 15);
-    const int fb = mr / M_T, m = mr - fb * M_T;  // row block, row in it
+  for (int f0 = 0; f0 < ROWS * COLS / 4; f0 += NTH) {
+    const int f = f0 + tid;  // float4 index: row f / (COLS / 4), columns 4 * (f % (COLS / 4)) ..
+    const int mr = f / (COLS / 4), n = 4 * (f % (COLS / 4));
+    const int fb = mr / M_T * CB + n / M_T, m = mr % M_T;  // block, row in it
     const long row = m0 + mr;
     if (row >= M) continue;
-    const float *rb0 = smem + (fb * NWK) * (M_T * M_T) + m * M_T + (n ^ swz(m));
+    const float *rb0 = smem + (fb * NWK) * (M_T * M_T) + m * M_T + (n % M_T ^ swz(m));
     float4 v = *reinterpret_cast<const float4 *>(rb0);
 #pragma unroll
     for (int w = 1; w < NWK; w++) {
@@ -1358,6 +1369,7 @@ constexpr int TILE_BK[NTILE] = {32, 32, 32, 32, 32, 32, 32, 32, 32, 64, 64};
 int g_force_tile = -1, g_force_splits = -1;
 int g_direct = 1;  // direct-to-LDS 256x256 kernel enabled (tth_gemm_direct)
 int g_mid = 1;     // 64x64 direct-load kernel for plain GEMMs (tth_gemm_mid; 2: shared k tiles)
+int g_large = 1;   // the plan of large plain GEMMs (ttk_gemm_large)
 int g_mid_force = 0;  // every plain GEMM of small size takes it too (tth_gemm_mid_force)
 int g_small = 1;   // 32x32 register kernel for small plain GEMMs (tth_gemm_small)
 int g_t16 = 1;     // 16x16 forward kernel for GEMMs below a full 32x32 grid (tth_gemm_t16)
@@ -2100,6 +2112,122 @@ int run_mid(int M, int N, int K, const Opnd &A, const Opnd &B, float *C, long ld
   return 0;
 }
 
+// The direct-load kernel on 128x128 tiles, one workgroup of eight waves (four
+// blocks x two k slices) a CU: half the loads a flop of the 64x64 tiles.
+constexpr int RT = 128;
+
+template <bool A_KC, bool B_NC, bool DW>
+int run_ring(int splits, int kc, int M, int N, int K, const Opnd &A, const Opnd &B, float *C,
+             long ldc) {
+  float *target = C, *ws = nullptr;
+  long tld = ldc;
+  if (splits > 1) {
+    ws = ws_alloc(sizeof(float) * (size_t)M * N * splits);
+    if (!ws) return -2;
+    target = ws;
+    tld = N;
+  }
+  const bool cvec = aligned16(target) && tld % 4 == 0;
+  const long tiles = (long)((M + RT - 1) / RT) * ((N + RT - 1) / RT);
+  hipLaunchKernelGGL((gemm_mid_kernel<A_KC, B_NC, 32, 4, 8, RT, 2, DW, false, RT>),
+                     dim3((unsigned)tiles, 1, splits), dim3(512), 0, stream(), M, N, K, A.p, A.ld,
+                     B.p, B.ld, target, tld, (long)M * N, kc, cvec, M, N);
+  int rc = hipGetLastError() == hipSuccess ? 0 : -3;
+  if (ws) {
+    if (rc == 0) rc = reduce_splits<EPI_STORE>(ws, C, M, N, splits, ldc, nullptr, 1);
+    ws_free(ws);
+  }
+  return rc;
+}
+
+// ---- the plan of a large plain GEMM ----
+// Estimated microseconds of each kernel on one block of C: whole rounds of
+// 256 CUs times a tile's K loop, at the per-k times measured (us a round and
+// k: 64x64 tiles 0.0185 alone on a CU, 0.040 two a CU and 0.018 for a last
+// half round (2048 x 1024 x 1024 39.3 us, 709 x 3052 x 1617 93); 128x128 0.064 (2048^3 136 us, 126 TFLOP/s, where register-staged
+// tiles took 155); 256x64 0.075; 256x256 0.2265; 4-byte loads 8-16 % more).
+// A grid a little over a round costs a whole one more, so the rows or columns
+// past the last full round may run as a GEMM of their own (4097 x 4095 x 4093:
+// 2541 us on 256x128 register-staged tiles; 1416 as one grid of 33 x 32 tiles;
+// as 32 x 32 and a row 1190).
+enum { PK_MID, PK_RING, PK_DIRECT };
+constexpr double PLAN_WS = TT_GEMM_SCRATCH_BYTES / 2.0;  // the split partials of one block, at most
+bool g_second = false;  // inside one of the two GEMMs
+struct BlockPlan {
+  int kind, splits, kc;
+  double us;
+};
+
+BlockPlan plan_block(int M, int N, int K, bool dw, bool direct_ok) {
+  const double CUS = 256;
+  int kc;
+  const int s = mid_splits(M, N, K, &kc);
+  const double n = ceil(M / 64.0) * ceil(N / 64.0) * s, kk = (double)(s > 1 ? kc : K);
+  const double red = s > 1 ? 4 + 8.0 * M * N * s / 3.5e6 : 0;
+  const double slow = dw ? 1.1 : 1.0;
+  BlockPlan p{PK_MID, s, kc, 0};
+  if (n <= CUS) {
+    p.us = slow * 0.0185 * kk + 3 + red;
+  } else {
+    const double rem = n - 512 * floor(n / 512);
+    p.us = kk * (0.040 * floor(n / 512) + (rem == 0 ? 0 : rem <= CUS ? 0.018 : 0.040)) + 4 + red;
+  }
+  const double tall = ceil(M / 256.0);
+  if (N <= M_T && s == 1 && tall >= CUS) p.us = slow * 0.075 * K * ceil(tall / CUS) + 4;
+  const double rt = ceil(M / 128.0) * ceil(N / 128.0);
+  for (int rs = 1; rs <= 4; rs *= 2) {
+    if (rs > 1 && (K / rs < 256 || 4.0 * M * N * rs > PLAN_WS)) break;
+    const int rkc = ((K + rs - 1) / rs + 63) / 64 * 64, rsp = (K + rkc - 1) / rkc;
+    // its waves sum half of K each, the 64x64 tiles' an eighth or a quarter:
+    // not over more than 2304 k a wave unless the grid is past those tiles'
+    if ((rsp > 1 ? rkc : K) > 4608 && rt < CUS) continue;
+    const double us = slow * 0.064 * (rsp > 1 ? rkc : K) * ceil(rt * rsp / CUS) + 5 +
+                      (rsp > 1 ? 4 + 8.0 * M * N * rsp / 3.5e6 : 0);
+    if (us < p.us) p = BlockPlan{PK_RING, rsp, rkc, us};
+  }
+  if (direct_ok && M % D_BM == 0 && N % D_BN == 0 && K % D_BK == 0) {
+    const double us = 0.2265 * K * ceil((M / 256) * (double)(N / 256) / CUS) + 5;
+    if (us < p.us) p = BlockPlan{PK_DIRECT, 1, K, us};
+  }
+  return p;
+}
+
+// Rows (or columns) m1 of the first of two GEMMs, or 0: one GEMM.
+struct LargePlan {
+  int m1, n1;
+};
+
+LargePlan plan_large(int M, int N, int K, bool dw, bool direct_ok) {
+  double best = plan_block(M, N, K, dw, direct_ok).us;
+  LargePlan p{0, 0};
+  const double rest = 12;  // a second, small GEMM at least (two launches)
+  auto rows = [&](int m1) {
+    if (m1 <= 0 || m1 >= M) return;
+    const double b = plan_block(M - m1, N, K, dw, false).us;
+    const double us = plan_block(m1, N, K, dw, direct_ok).us + (b > rest ? b : rest);
+    if (us < best) { best = us; p = LargePlan{m1, 0}; }
+  };
+  auto cols = [&](int n1) {
+    if (n1 <= 0 || n1 >= N) return;
+    const double b = plan_block(M, N - n1, K, dw, false).us;
+    const double us = plan_block(M, n1, K, dw, direct_ok).us + (b > rest ? b : rest);
+    if (us < best) { best = us; p = LargePlan{0, n1}; }
+  };
+  // (tt_k_gemm_noalloc takes the same plan and launches only once all of its
+  // workspace is certain to fit its scratch)
+  auto fits = [&](int m, int n) {
+    return 4.0 * m * n * plan(m, n, K).splits <= PLAN_WS;
+  };
+  const long tm = (M + 127) / 128, tn = (N + 127) / 128, full = tm * tn / 256 * 256;
+  rows((int)(full / tn) * 128);
+  cols((int)(full / tm) * 128);
+  rows(M / 64 * 64);
+  cols(N / 64 * 64);
+  rows(M / 256 * 256);
+  if ((p.m1 && !fits(M - p.m1, N)) || (p.n1 && !fits(M, N - p.n1))) p = LargePlan{0, 0};
+  return p;
+}
+
 template <bool A_KC, bool A_PERM, bool B_NC, bool B_PERM, int EPI, bool B_I2C = false>
 int run(int M, int N, int K, Opnd A, Opnd B, float *C, long ldc, const float *bias, int HW,
         bool vec, const I2C &cv = I2C{}) {
@@ -2107,6 +2235,62 @@ int run(int M, int N, int K, Opnd A, Opnd B, float *C, long ldc, const float *bi
   // K == 0 runs no K tiles: the epilogue stores zeros (plus bias)
   Plan p = plan(M, N, K > 0 ? K : 1);
   if constexpr (!A_PERM && !B_PERM && !B_I2C && EPI == EPI_STORE) {
+    // from 0.5 GFLOP: the kernel, split and, past the last full round of
+    // tiles, the second GEMM that plan_large picks
+    const bool large = 2.0 * M * N * K >= (double)(1L << 29) && N > 16 && M > 16;
+    if (((large && g_large && g_mid == 1 && !g_mid_force) || g_large == 2) && g_force_tile < 0 &&
+        g_force_splits < 0 && K > 0 && A.ld <= (1L << 22) && B.ld <= (1L << 22) &&
+        !(g_large == 1 && small_ok<A_KC, B_NC>(M, N, K, A, B))) {
+      const bool v = vec && (!(A_KC || !B_NC) || K % 4 == 0) && (A_KC || M % 4 == 0) &&
+                     (!B_NC || N % 4 == 0);
+      const bool dok = g_direct && vec && aligned16(C) && ldc % 4 == 0;
+      const LargePlan lp = g_large == 2 || g_second ? LargePlan{0, 0} : plan_large(M, N, K, !v, dok);
+      // the two GEMMs are not split again, and an epilogue that wants all of C
+      // at once is left to its own pass
+      struct Nest {
+        bool second;
+        RedHook *hook;
+        explicit Nest(bool on) : second(g_second), hook(g_red_hook) {
+          g_second = second || on;
+          if (on) g_red_hook = nullptr;
+        }
+        ~Nest() {
+          g_second = second;
+          g_red_hook = hook;
+        }
+      } nest(lp.m1 || lp.n1);
+      if (lp.m1) {
+        Opnd A2 = A;
+        A2.p += A_KC ? lp.m1 * A.ld : lp.m1;
+        const int rc = run<A_KC, A_PERM, B_NC, B_PERM, EPI, B_I2C>(lp.m1, N, K, A, B, C, ldc, bias,
+                                                                 HW, vec);
+        return rc ? rc
+                  : run<A_KC, A_PERM, B_NC, B_PERM, EPI, B_I2C>(
+                        M - lp.m1, N, K, A2, B, C + lp.m1 * ldc, ldc, bias, HW,
+                        vec && aligned16(A2.p));
+      }
+      if (lp.n1) {
+        Opnd B2 = B;
+        B2.p += B_NC ? lp.n1 : lp.n1 * B.ld;
+        const int rc = run<A_KC, A_PERM, B_NC, B_PERM, EPI, B_I2C>(M, lp.n1, K, A, B, C, ldc, bias,
+                                                                 HW, vec);
+        return rc ? rc
+                  : run<A_KC, A_PERM, B_NC, B_PERM, EPI, B_I2C>(M, N - lp.n1, K, A, B2, C + lp.n1,
+                                                              ldc, bias, HW,
+                                                              vec && aligned16(B2.p));
+      }
+      const BlockPlan bp = g_large == 2 ? BlockPlan{PK_RING, 1, (K + 63) / 64 * 64, 0}
+                                        : plan_block(M, N, K, !v, dok);
+      if (bp.kind == PK_RING)
+        return v ? run_ring<A_KC, B_NC, false>(bp.splits, bp.kc, M, N, K, A, B, C, ldc)
+                 : run_ring<A_KC, B_NC, true>(bp.splits, bp.kc, M, N, K, A, B, C, ldc);
+      if (bp.kind == PK_MID)
+        return v ? run_mid<A_KC, B_NC>(M, N, K, A, B, C, ldc)
+                 : run_mid<A_KC, B_NC, true>(M, N, K, A, B, C, ldc);
+      p.tile = T256x256;  // whole 256x256 tiles: the direct-load kernel below
+      p.splits = 1;
+      p.kchunk = K;
+    }
     if (p.tile != T256x256 && p.tile != T256x128 && p.tile != T128x128 && g_force_tile < 0) {
       if (!g_mid_force && small_ok<A_KC, B_NC>(M, N, K, A, B))
         return run_small<A_KC, B_NC>(M, N, K, A, B, C, ldc);
@@ -2232,6 +2416,14 @@ extern "C" int tth_gemm_direct(int on) {
 extern "C" int tth_gemm_mid(int on) {
   g_mid = on == 2 ? 2 : on ? 1 : 0;
   return 0;
+}
+
+// Tuning and tests: 0 keeps plain GEMMs from the plan below (the smaller
+// kernels' own rules), 2 sends every one of them to the 128x128 tiles.
+extern "C" int ttk_gemm_large(int on) {
+  const int prev = g_large;
+  if (on >= 0) g_large = on;
+  return prev;
 }
 
 extern "C" int tth_gemm_mid_force(int on) {
