@@ -283,6 +283,12 @@ static const Tensor *padones_input(const AGNode *a) {
                                                                                        : NULL;
 }
 
+/* A layer wide enough that its padded input is not worth writing: the weight
+ * gradient is formed from the unpadded one (rows of K floats are aligned where
+ * rows of K + 1 are not: 2049 x 1024 x 1000 from [X, 1] 51 us in two GEMMs, from
+ * X 41 and the bias row 3), and the padded tensor is a recipe. */
+static int pad_unwritten(long M, long K) { return M * K >= 1L << 18; }
+
 AGNode *ag_matmul(AGNode *a, AGNode *b) {
     if (!a || !b) return NULL;
     const Tensor *av = a->val, *bv = b->val;
@@ -456,6 +462,11 @@ AGNode *ag_padones(AGNode *a) {
         if (v) {
             const TTPendConv p = tt_pend;
             tt_pend.active = 0;
+            if (p.b && pad_unwritten(M, K) &&
+                ttk_gemm_bias_relu(p.geo[0], p.geo[1], p.geo[2], p.x, p.w, p.b, p.out->dev,
+                                   p.r->dev) == 0 &&
+                (tt_lazy_padones(v, a->val) == 0 || tt_k_padones_fwd(p.r->dev, v->dev, M, K) == 0))
+                return make_node(v, &OP_PADONES, a, NULL, NULL);
             if ((p.b ? tt_k_gemm_bias_relu_pad(p.geo[0], p.geo[1], p.geo[2], p.x, p.w, p.b,
                                                p.out->dev, p.r->dev, v->dev)
                      : tt_k_gemm_relu_pad(p.geo[0], p.geo[1], p.geo[2], p.x, p.w, p.out->dev,
@@ -788,6 +799,9 @@ static int backward_matmul_fused(AGNode *n, const float *g, const TTHeadCeArgs *
     const int head = N <= HEAD_MAX_N;
     if (!head && !(needs(a) && needs(b))) return -1;
     if (ce && !head) return -1;
+    /* past both kernels' sizes: nothing is read (the padded input may be a
+     * recipe) */
+    if (head ? needs(b) && M > 480 : 2.0 * M * N * K >= (double)(1L << 29)) return -1;
     const float *ad = needs(b) ? tt_dev(a->val) : NULL;
     const float *bd = needs(a) ? tt_dev(b->val) : NULL;
     if ((needs(b) && !ad) || (needs(a) && !bd)) return -1;
@@ -961,6 +975,17 @@ static void backward_matmul(AGNode *n) {
         Tensor *ga = bd ? tt_empty_like(a->val) : NULL;
         if (ga && tt_k_gemm(M, K, N, g, N, 0, bd, N, 1, ga->dev, K) == 0) accum_move(a, ga);
         else tt_release(ga);
+    }
+    /* (a padded value that the host holds may have been changed there) */
+    const Tensor *xp = needs(b) && K > 1 && pad_unwritten(M, K - 1) && a->val->valid & TT_V_DEV
+                           ? padones_input(a)
+                           : NULL;
+    if (xp) {  /* dB from the padones input */
+        const float *xd = tt_dev((Tensor *)xp);
+        Tensor *gb = xd ? tt_empty_like(b->val) : NULL;
+        if (gb && ttk_gemm_tn_colsum(M, K - 1, N, xd, g, gb->dev) == 0) accum_move(b, gb);
+        else tt_release(gb);
+        return;
     }
     if (needs(b)) {  /* dB = a^T (a is MxK) * g (MxN) */
         const float *ad = tt_dev(a->val);

@@ -1083,6 +1083,39 @@ __global__ void bias_relu_pad_rows_kernel(float *__restrict__ c, const float *__
   }
 }
 
+// 16 columns a workgroup, 64 row lanes a column: bound by the read of g (1000
+// x 1024: 4 MB)
+__global__ void __launch_bounds__(1024)
+colsum_kernel(const float *__restrict__ g, float *__restrict__ out, int M, int N) {
+  __shared__ float part[64][17];
+  const int c = threadIdx.x & 15, r = threadIdx.x >> 4;
+  const int n = blockIdx.x * 16 + c;
+  float v = 0.0f;
+  if (n < N) {
+    int m = r;
+    for (; m + 192 < M; m += 256) {
+      const float a = g[(long)m * N + n], b = g[(long)(m + 64) * N + n];
+      const float d = g[(long)(m + 128) * N + n], e = g[(long)(m + 192) * N + n];
+      v += a; v += b; v += d; v += e;
+    }
+    for (; m < M; m += 64) v += g[(long)m * N + n];
+  }
+  part[r][c] = v;
+  __syncthreads();
+  for (int o = 32; o > 0; o >>= 1) {
+    if (r < o) part[r][c] += part[r + o][c];
+    __syncthreads();
+  }
+  if (r == 0 && n < N) out[n] = part[0][c];
+}
+
+extern "C" int ttk_colsum(const float *g, float *out, int M, int N) {
+  if (M <= 0 || N <= 0 || !g || !out) return -1;
+  hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((N + 15) / 16)), dim3(1024), 0, stream(), g, out,
+                     M, N);
+  return launched();
+}
+
 extern "C" int ttk_bias_relu_pad(float *c, const float *bias, float *r, float *p, int M, int N) {
   if (M <= 0 || N <= 0) return 0;
   if (M >= 65536) return -1;

@@ -1087,6 +1087,13 @@ struct MidOperand {
   }
 };
 
+// A matmul layer's epilogue: C = A B + bias and r = relu(C), rows of ldc (r
+// null: none).
+struct MidEpi {
+  const float *bias;
+  float *r;
+};
+
 // ROWS: rows of A per tile (64, or 256 for tall operands with few columns:
 // four 64-row blocks share each tile of B); NWK: waves per K tile.  Wave w
 // owns row block w / NWK and k slice w % NWK.  PRIV (one row block, BK = 8 NW):
@@ -1098,11 +1105,11 @@ struct MidOperand {
 // COLS: columns of B per tile (64 or 128): wave w owns 64x64 block w / NWK of
 // the tile's ROWS / 64 x COLS / 64.
 template <bool A_KC, bool B_NC, int BK, int S, int NW, int ROWS = M_T, int NWK = NW,
-          bool DW = false, bool PRIV = false, int COLS = M_T>
+          bool DW = false, bool PRIV = false, int COLS = M_T, bool EPI = false>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4, 2)))
 gemm_mid_kernel(int M, int N, int K, const float *__restrict__ A, long lda,
                 const float *__restrict__ B, long ldb, float *__restrict__ C, long ldc,
-                long split_stride, int kchunk, bool cvec, int alim, int blim) {
+                long split_stride, int kchunk, bool cvec, int alim, int blim, MidEpi epi) {
   TT_PROBE(0, 0);
   static_assert(S >= 3, "the pipeline needs three stages");
   constexpr int NTH = 64 * NW;
@@ -1133,8 +1140,11 @@ gemm_mid_kernel(int M, int N, int K, const float *__restrict__ A, long lda,
   const int tiles_m = (M + ROWS - 1) / ROWS, tiles_n = (N + COLS - 1) / COLS;
   const int ntiles = tiles_m * tiles_n;
   int pid = blockIdx.x;
-  {
-    // neighbouring tiles on one XCD: the first ntiles % 8 XCDs take one more
+  // neighbouring tiles on one XCD
+  if constexpr (COLS == M_T) {
+    if ((ntiles & 7) == 0) pid = (pid & 7) * (ntiles >> 3) + (pid >> 3);
+  } else {
+    // the first ntiles % 8 XCDs take one more
     const int q = ntiles >> 3, xcd = pid & 7;
     pid = xcd * q + min(xcd, ntiles & 7) + (pid >> 3);
   }
@@ -1299,6 +1309,34 @@ gemm_mid_kernel(int M, int N, int K, const float *__restrict__ A, long lda,
   TT_PROBE(0, 3);
   __syncthreads();
   TT_PROBE(0, 4);
+  // EPI: the epilogue of a layer and rows that are not 16-byte aligned, the
+  // latter a lane an element, so that a store's lanes are consecutive (four
+  // consecutive floats a lane, one by one, took 1000 x 2048 x 1024 into rows
+  // of 2049 floats from 34 to 48 us).  An instance of its own: in the plain
+  // one the longer code cost 1024^3 1.5 % (21.5 -> 21.85 us).
+  if constexpr (EPI) {
+    if (!cvec) {
+#pragma unroll 4
+      for (int f0 = 0; f0 < ROWS * COLS; f0 += NTH) {
+        const int f = f0 + tid;
+        const int mr = f / COLS, n = f % COLS;
+        const int fb = mr / M_T * CB + n / M_T, m = mr % M_T;
+        const long row = m0 + mr, col = n0 + n;
+        if (row >= M || col >= N) continue;
+        const float *rb0 = smem + (fb * NWK) * (M_T * M_T) + m * M_T + (n % M_T ^ swz(m));
+        float v = rb0[0];
+#pragma unroll
+        for (int w = 1; w < NWK; w++) v += rb0[w * (M_T * M_T)];
+        if (epi.r) {
+          v += epi.bias[col];
+          epi.r[row * ldc + col] = v > 0.f ? v : 0.f;
+        }
+        C[row * ldc + col] = v;
+      }
+      TT_PROBE(0, 5);
+      return;
+    }
+  }
 #pragma unroll
   for (int f0 = 0; f0 < ROWS * COLS / 4; f0 += NTH) {
     const int f = f0 + tid;  // float4 index: row f / (COLS / 4), columns 4 * (f % (COLS / 4)) ..
@@ -1315,6 +1353,26 @@ gemm_mid_kernel(int M, int N, int K, const float *__restrict__ A, long lda,
     }
     float *crow = C + row * ldc;
     const long col = n0 + n;
+    if constexpr (EPI) {
+      if (epi.r) {
+        float x[4] = {v.x, v.y, v.z, v.w};
+        float r[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          x[i] += epi.bias[min(col + i, (long)N - 1)];
+          r[i] = x[i] > 0.f ? x[i] : 0.f;
+        }
+        v = make_float4(x[0], x[1], x[2], x[3]);
+        float *rrow = epi.r + row * ldc;
+        if (col + 3 < N) {
+          *reinterpret_cast<float4 *>(rrow + col) = make_float4(r[0], r[1], r[2], r[3]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            if (col + i < N) rrow[col + i] = r[i];
+        }
+      }
+    }
     if (cvec && col + 3 < N) {
       *reinterpret_cast<float4 *>(crow + col) = v;
     } else {
@@ -2058,7 +2116,8 @@ int mid_splits(int M, int N, int K, int *kc_out) {
 
 // DW: 4-byte loads (operands of any alignment and row length, read in place).
 template <bool A_KC, bool B_NC, bool DW = false>
-int run_mid(int M, int N, int K, const Opnd &A, const Opnd &B, float *C, long ldc) {
+int run_mid(int M, int N, int K, const Opnd &A, const Opnd &B, float *C, long ldc,
+            const MidEpi &epi = MidEpi{}) {
   const int CUS = 256;
   const long tiles = (long)((M + M_T - 1) / M_T) * ((N + M_T - 1) / M_T);
   int kc;
@@ -2072,7 +2131,8 @@ int run_mid(int M, int N, int K, const Opnd &A, const Opnd &B, float *C, long ld
     target = ws;
     tld = N;
   }
-  const bool cvec = aligned16(target) && tld % 4 == 0;
+  const bool cvec = aligned16(target) && tld % 4 == 0 && (!epi.r || aligned16(epi.r));
+  const bool x = !cvec || epi.r;  // the extended stores
   const dim3 grid((unsigned)tiles, 1, splits);
   const long sstride = (long)M * N;
   // at most one workgroup per CU: 8 waves (two per SIMD), a ring of 4
@@ -2081,27 +2141,32 @@ int run_mid(int M, int N, int K, const Opnd &A, const Opnd &B, float *C, long ld
   // the waves (64-k stages, 4 of them, and 32-k stages, 5 of them)
   const int alim = M, blim = N;
   const long tiles256 = (long)((M + 255) / 256) * ((N + M_T - 1) / M_T);
-  if (N <= M_T && splits == 1 && tiles256 >= CUS)
+#define TT_MID_X(EXT, PLAIN, NTHR)                                                              \
+  {                                                                                             \
+    auto kern = x ? EXT : PLAIN;                                                                \
+    hipLaunchKernelGGL(kern, grid, dim3(NTHR), 0, stream(), M, N, K, A.p, A.ld, B.p, B.ld,      \
+                       target, tld, sstride, kc, cvec, alim, blim, epi);                        \
+  }
+  if (!epi.r && N <= M_T && splits == 1 && tiles256 >= CUS)
     // tall: 256-row tiles, the 64 columns of B loaded once for four row blocks
     hipLaunchKernelGGL((gemm_mid_kernel<A_KC, B_NC, 32, 4, 8, 256, 2, DW>),
                        dim3((unsigned)tiles256), dim3(512), 0, stream(), M, N, K, A.p, A.ld, B.p,
-                       B.ld, target, tld, sstride, kc, cvec, alim, blim);
+                       B.ld, target, tld, sstride, kc, cvec, alim, blim, epi);
   else if (tiles * splits <= CUS && g_mid != 2)
-    hipLaunchKernelGGL((gemm_mid_kernel<A_KC, B_NC, 64, 4, 8, M_T, 8, DW, true>), grid, dim3(512),
-                       0, stream(), M, N, K, A.p, A.ld, B.p, B.ld, target, tld, sstride, kc, cvec,
-                       alim, blim);
+    TT_MID_X((gemm_mid_kernel<A_KC, B_NC, 64, 4, 8, M_T, 8, DW, true, M_T, true>),
+             (gemm_mid_kernel<A_KC, B_NC, 64, 4, 8, M_T, 8, DW, true>), 512)
   else if (tiles * splits <= CUS)
     hipLaunchKernelGGL((gemm_mid_kernel<A_KC, B_NC, 64, 4, 8, M_T, 8, DW>), grid, dim3(512), 0,
                        stream(), M, N, K, A.p, A.ld, B.p, B.ld, target, tld, sstride, kc, cvec,
-                       alim, blim);
+                       alim, blim, epi);
   else if (g_mid != 2)
-    hipLaunchKernelGGL((gemm_mid_kernel<A_KC, B_NC, 32, 4, 4, M_T, 4, DW, true>), grid, dim3(256),
-                       0, stream(), M, N, K, A.p, A.ld, B.p, B.ld, target, tld, sstride, kc, cvec,
-                       alim, blim);
+    TT_MID_X((gemm_mid_kernel<A_KC, B_NC, 32, 4, 4, M_T, 4, DW, true, M_T, true>),
+             (gemm_mid_kernel<A_KC, B_NC, 32, 4, 4, M_T, 4, DW, true>), 256)
   else
     hipLaunchKernelGGL((gemm_mid_kernel<A_KC, B_NC, 32, 5, 4, M_T, 4, DW>), grid, dim3(256), 0,
                        stream(), M, N, K, A.p, A.ld, B.p, B.ld, target, tld, sstride, kc, cvec,
-                       alim, blim);
+                       alim, blim, epi);
+#undef TT_MID_X
   const bool own = ws != nullptr;
   if (hipGetLastError() != hipSuccess) { if (own) ws_free(ws); return -3; }
   if (ws) {
@@ -2118,7 +2183,7 @@ constexpr int RT = 128;
 
 template <bool A_KC, bool B_NC, bool DW>
 int run_ring(int splits, int kc, int M, int N, int K, const Opnd &A, const Opnd &B, float *C,
-             long ldc) {
+             long ldc, const MidEpi &epi = MidEpi{}) {
   float *target = C, *ws = nullptr;
   long tld = ldc;
   if (splits > 1) {
@@ -2127,11 +2192,12 @@ int run_ring(int splits, int kc, int M, int N, int K, const Opnd &A, const Opnd 
     target = ws;
     tld = N;
   }
-  const bool cvec = aligned16(target) && tld % 4 == 0;
+  const bool cvec = aligned16(target) && tld % 4 == 0 && (!epi.r || aligned16(epi.r));
   const long tiles = (long)((M + RT - 1) / RT) * ((N + RT - 1) / RT);
-  hipLaunchKernelGGL((gemm_mid_kernel<A_KC, B_NC, 32, 4, 8, RT, 2, DW, false, RT>),
-                     dim3((unsigned)tiles, 1, splits), dim3(512), 0, stream(), M, N, K, A.p, A.ld,
-                     B.p, B.ld, target, tld, (long)M * N, kc, cvec, M, N);
+  auto kern = !cvec || epi.r ? gemm_mid_kernel<A_KC, B_NC, 32, 4, 8, RT, 2, DW, false, RT, true>
+                             : gemm_mid_kernel<A_KC, B_NC, 32, 4, 8, RT, 2, DW, false, RT>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)tiles, 1, splits), dim3(512), 0, stream(), M, N, K, A.p, A.ld,
+                     B.p, B.ld, target, tld, (long)M * N, kc, cvec, M, N, epi);
   int rc = hipGetLastError() == hipSuccess ? 0 : -3;
   if (ws) {
     if (rc == 0) rc = reduce_splits<EPI_STORE>(ws, C, M, N, splits, ldc, nullptr, 1);
@@ -2281,6 +2347,21 @@ int run(int M, int N, int K, Opnd A, Opnd B, float *C, long ldc, const float *bi
       }
       const BlockPlan bp = g_large == 2 ? BlockPlan{PK_RING, 1, (K + 63) / 64 * 64, 0}
                                         : plan_block(M, N, K, !v, dok);
+      if constexpr (A_KC && B_NC) {
+        // a layer's bias and relu in the tiles' stores
+        RedHook *const h = g_red_hook;
+        if (h && h->kind == HOOK_RELU_PAD && h->C == C && ldc == N && h->rp.bias && h->rp.r &&
+            !h->rp.p && bp.splits == 1 && bp.kind != PK_DIRECT && g_mid != 2 &&
+            !(bp.kind == PK_MID && N <= M_T)) {
+          const MidEpi e{h->rp.bias, h->rp.r};
+          h->applied = 1;
+          if (bp.kind == PK_RING)
+            return v ? run_ring<A_KC, B_NC, false>(1, bp.kc, M, N, K, A, B, C, ldc, e)
+                     : run_ring<A_KC, B_NC, true>(1, bp.kc, M, N, K, A, B, C, ldc, e);
+          return v ? run_mid<A_KC, B_NC, false>(M, N, K, A, B, C, ldc, e)
+                   : run_mid<A_KC, B_NC, true>(M, N, K, A, B, C, ldc, e);
+        }
+      }
       if (bp.kind == PK_RING)
         return v ? run_ring<A_KC, B_NC, false>(bp.splits, bp.kc, M, N, K, A, B, C, ldc)
                  : run_ring<A_KC, B_NC, true>(bp.splits, bp.kc, M, N, K, A, B, C, ldc);
@@ -2658,6 +2739,32 @@ extern "C" int tt_k_gemm_bias_relu_pad(int M, int N, int K, const float *A, cons
   g_red_hook = nullptr;
   if (rc) return rc;
   return h.applied ? 0 : ttk_bias_relu_pad(C, bias, R, P, M, N);
+}
+
+// C = A * B + bias and R = relu(C) for a layer of at least 2^29 flops (the
+// values of tt_k_gemm_bias_relu_pad), in the tiles' stores where the plan is
+// one unsplit kernel.  1: smaller, nothing launched.
+extern "C" int ttk_gemm_bias_relu(int M, int N, int K, const float *A, const float *B,
+                                  const float *bias, float *C, float *R) {
+  if (M <= 0 || N <= 16 || K <= 0 || 2.0 * M * N * K < (double)(1L << 29) || g_force_tile >= 0)
+    return 1;
+  RedHook h{};
+  h.kind = HOOK_RELU_PAD;
+  h.C = C;
+  h.rp = ReluPadEx{R, nullptr, bias};
+  g_red_hook = &h;
+  const int rc = tt_k_gemm(M, N, K, A, K, 0, B, N, 0, C, N);
+  g_red_hook = nullptr;
+  if (rc) return rc;
+  return h.applied ? 0 : ttk_bias_relu_pad(C, bias, R, nullptr, M, N);
+}
+
+// dW = [X, 1]^T * G ((Kx + 1) x N) of a large layer from X itself: the product
+// with X's aligned rows, and the last row the column sums of G.
+extern "C" int ttk_gemm_tn_colsum(int rows, int Kx, int N, const float *X, const float *G,
+                                  float *dW) {
+  const int rc = tt_k_gemm(Kx, N, rows, X, Kx, 1, G, N, 0, dW, N);
+  return rc ? rc : ttk_colsum(G, dW + (long)Kx * N, rows, N);
 }
 
 // C = A * B + bias as tt_k_gemm_bias_relu_pad (C only) and, when the GEMM

@@ -43,6 +43,15 @@ int    ttk_add_outside(float *c, const float *cin, int M, int N, int mb, int nb)
 /* elementwise.hip: c[m][n] += bias[n] for the M x N matrix c, and when r / p
  * are given r = relu(c), p = [r, 1] (M x N+1) */
 int    ttk_bias_relu_pad(float *c, const float *bias, float *r, float *p, int M, int N);
+/* elementwise.hip: out[n] = the sum of column n of the M x N matrix g, rows
+ * dealt to 64 lanes a column and their sums added in a fixed tree */
+int    ttk_colsum(const float *g, float *out, int M, int N);
+/* gemm.hip: a large layer's product, bias and relu, and its weight gradient
+ * from the unpadded input */
+int    ttk_gemm_bias_relu(int M, int N, int K, const float *A, const float *B, const float *bias,
+                          float *C, float *R);
+int    ttk_gemm_tn_colsum(int rows, int Kx, int N, const float *X, const float *G, float *dW);
+int    ttk_gemm_large(int on);          /* tuning: the plan of large GEMMs */
 /* elementwise.hip: the split-K reduction of a GEMM (ws: S partial M x N
  * products, summed as gemm.hip's reduce_one does with zl lanes an element)
  * plus bias into C, and the softmax-CE of C's rows in the same launch:
