@@ -326,6 +326,38 @@ def test_conv_chain_bwd_matches_separate(tlib, N, C1):
     assert np.abs(fb.to_np((32,)) - rdb).max() <= 1e-4 * max(1.0, np.abs(rdb).max())
 
 
+@pytest.mark.parametrize("B,C1", [(1, 3), (43, 1), (80, 2), (127, 3), (257, 3)])
+def test_autograd_chain_bwd_any_batch(tlib, B, C1):
+    """The one-launch backward at batches whose separate weight gradient sums
+    other units of rows (below 128 and from 256 on): the filters' gradients of
+    the two orders of the same fp32 sums agree to the suite's fp32 bar, 1e-4
+    of the largest value (n = B * 1024 terms in random order: sqrt(n) * 2^-24
+    of the terms' scale, 3e-5 at n = 257 * 1024)."""
+    from tinytorch_amd.torch_py import Node
+    r = np.random.default_rng(31 + B)
+    x, y, P = orc.cnn_inputs(B=B)
+    x = r.uniform(0, 1, (B, C1, 32, 32)).astype(np.float32)
+    P = dict(P, w1=(r.standard_normal((32, C1, 3, 3)) * 0.3).astype(np.float32))
+
+    def run(chain):
+        prev = tlib.tth_conv_chain(1 if chain else 0)
+        keep = []
+        try:
+            loss = _cnn(Node, x, P, keep).softmax_ce(y)
+            loss.backward(None)
+            g = [keep[i].grad() for i in range(1, 5)]  # w1, b1, w2, b2
+            for nd in [loss] + keep[::-1]:
+                nd.release()
+            return g
+        finally:
+            tlib.tth_conv_chain(prev)
+
+    print("chain bwd, B", B, "C1", C1, flush=True)
+    for a, b in zip(run(True), run(False)):
+        assert np.isfinite(a).all()
+        assert np.abs(a - b).max() <= 1e-4 * max(1e-30, np.abs(b).max())
+
+
 @pytest.mark.parametrize("when", ["before", "never", "after"])
 def test_autograd_chain_softmax_ce_recipe(tlib, when):
     """The config-4 graph with the chain's classifier partial sums: the

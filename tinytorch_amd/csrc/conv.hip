@@ -2424,8 +2424,8 @@ conv_chain_fwd_kernel(const float *__restrict__ x, const float *__restrict__ w1,
 //     backward: the window's gradient at its first argmax when that relu
 //     value is > 0, else zero);
 //   phase 3: the weight gradient of two units of 8 rows, four waves a unit,
-//     as conv_dwt_kernel<1, 1, true> (the same items, MFMA order, LDS sum
-//     (0 + 2) + (1 + 3) and bias sum), one partial block a unit.
+//     as conv_dwt_kernel<1, 1, true> with such units (the same items, MFMA
+//     order, LDS sum (0 + 2) + (1 + 3) and bias sum), one partial block a unit.
 namespace chainb {
 constexpr int NTH = 512;
 constexpr int G2 = 8, RS2 = 16 + G2, R2 = 10, CS2 = R2 * RS2 + 4;   // dc2 slab
@@ -3016,21 +3016,21 @@ extern "C" int tt_k_conv2d_chain_fwd(const float *x, const float *w1, const floa
 // bit for bit tt_k_conv2d_dx_lds; then the first convolution's (x N x C1 x
 // 32 x 32, C1 <= 3, 32 filters, 3x3, pad 1) weight and bias gradient from
 // dx2 through the 2x2 pool + relu backward of codes1, as the deferred
-// reduction *job (the partials tt_k_conv2d_dw_lds_pooled would reduce, the
-// same values).  -1: not covered (nothing launched); < -1: error.
+// reduction *job (units of 8 rows: for 128 <= N < 256 the partials
+// tt_k_conv2d_dw_lds_pooled would reduce, the same values).  Every batch up
+// to 1024 takes it: one launch for three, without dx2's second pass.  A
+// training step with it and with the three kernels: N = 64 58.6 against 75.8
+// us, 80 68.5 / 89.2, 110 72.8 / 82.1, 300 167 / 199, 512 257 / 280.
+// -1: not covered (nothing launched); < -1: error.
 extern "C" int ttk_conv2d_chain_bwd(const float *dc2, const float *w2, const unsigned char *codes1,
                                     const float *x, float *dx2, float *dw1, float *db1, int N,
                                     int C1, TTDwtJob *job, const float *x2, float *dw2,
                                     float *db2, TTDwtJob *job2) {
   if (!dc2 || !w2 || !codes1 || !x || !dx2 || !dw1 || !job || !g_dwt || N <= 0 ||
-      N > 16383 || C1 < 1 || C1 > 3)
+      N > 1024 || C1 < 1 || C1 > 3)
     return -1;
   if (!aligned16(dc2) || !aligned16(w2) || !aligned16(x) || ((uintptr_t)codes1 & 15)) return -1;
-  // the partials must be those of the plan tt_k_conv2d_dw_lds_pooled takes
-  const Geo g1{C1, 32, 32, 3, 3, 1, 1, 1, 1, 32, 32, 32, C1 * 9};
-  const DwtPlan tp = plan_dwt(g1, N);
-  if (tp.tg != 1 || tp.ntgw != 1 || tp.nts != 1 || tp.nfb != 1 || tp.rc != 8 || tp.jbp != 1)
-    return -1;
+  const int units = 4 * N;  // partials of the first weight gradient: 8 rows each
   // the second convolution's weight gradient in the same grid: its plan must
   // be the 3 x 3 tap-group kernel over whole images
   const Geo g2{32, 16, 16, 3, 3, 1, 1, 1, 1, 16, 16, 64, 288};
@@ -3046,7 +3046,7 @@ extern "C" int ttk_conv2d_chain_bwd(const float *dc2, const float *w2, const uns
   const void *kern = dw2 ? (const void *)conv_chain_bwd_dw2_kernel : (const void *)conv_chain_bwd_kernel;
   if (!allow_big_lds(kern)) return -1;
   const long S = 1024 + 32;
-  float *part = (float *)ttrt_alloc(sizeof(float) * (size_t)(S * tp.units));
+  float *part = (float *)ttrt_alloc(sizeof(float) * (size_t)(S * units));
   if (!part) return -2;
   float *part2 = nullptr;
   const long S2 = dw2 ? (long)t2.jbp * 1024 + 32 : 0;
@@ -3076,8 +3076,8 @@ extern "C" int ttk_conv2d_chain_bwd(const float *dc2, const float *w2, const uns
   }
   const long cols = S / 4;
   int zl = 1;
-  while (zl < 64 && zl * DWT_UPL < tp.units) zl *= 2;
-  *job = TTDwtJob{part, dw1, db1, tp.units, 1, 1, 32, C1 * 9, zl,
+  while (zl < 64 && zl * DWT_UPL < units) zl *= 2;
+  *job = TTDwtJob{part, dw1, db1, units, 1, 1, 32, C1 * 9, zl,
                   (int)((cols + NT / zl - 1) / (NT / zl))};
   return 0;
 }
@@ -3088,6 +3088,13 @@ extern "C" int tt_k_conv2d_chain_bwd(const float *dc2, const float *w2,
                                      const unsigned char *codes1, const float *x, float *dx2,
                                      float *dw1, float *db1, const float *x2, float *dw2,
                                      float *db2, int N, int C1) {
+  // promised bit for bit the separate weight gradient's values, which sums 8
+  // rows a unit at these batches only
+  const Geo g1{C1, 32, 32, 3, 3, 1, 1, 1, 1, 32, 32, 32, C1 * 9};
+  if (N <= 0 || C1 < 1 || C1 > 3) return -1;
+  const DwtPlan tp = plan_dwt(g1, N);
+  if (tp.tg != 1 || tp.ntgw != 1 || tp.nts != 1 || tp.nfb != 1 || tp.rc != 8 || tp.jbp != 1)
+    return -1;
   TTDwtJob job[2];
   const int rc = ttk_conv2d_chain_bwd(dc2, w2, codes1, x, dx2, dw1, db1, N, C1, &job[0], x2, dw2,
                                       db2, &job[1]);

@@ -100,8 +100,8 @@ int    ttk_conv2d_dwt_defer(const float *gr, const unsigned char *codes, const f
                             float *dw, float *db, const int geo[13], TTDwtJob *job);
 /* conv.hip: the CNN chain's middle backward in one launch: dx2 = the input
  * gradient of the second convolution (tt_k_conv2d_dx_lds bits) and the first
- * convolution's weight gradient through the pool codes1 (the job
- * tt_k_conv2d_dw_lds_pooled would defer); with dw2 (db2 optional), the
+ * convolution's weight gradient through the pool codes1 (partials of 8 output
+ * rows, a job as tt_k_conv2d_dw_lds_pooled would defer); with dw2 (db2 optional), the
  * second convolution's weight gradient from dc2 and its input x2 in the same
  * grid (the job tt_k_conv2d_dw_lds would defer, *job2).  -1: not covered. */
 int    ttk_conv2d_chain_bwd(const float *dc2, const float *w2, const unsigned char *codes1,
