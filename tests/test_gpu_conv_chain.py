@@ -132,6 +132,49 @@ def test_conv_chain_matches_two_launches(tlib, N, C1, bias, nan):
     assert bits_equal(s2.to_np((N, 64, 8, 8)), orc.maxpool_fwd(orc.relu_fwd(y2), 2, 2, 2, 2))
 
 
+# more than 256 image halves: a workgroup takes several (two, the last one of
+# some missing; two of 193; three with all optional outputs and NaN inputs; five)
+@pytest.mark.parametrize("N,C1,bias,nan", [(129, 3, True, False), (193, 1, False, False),
+                                           (259, 4, True, True), (600, 2, True, False)])
+def test_conv_chain_many_halves(tlib, N, C1, bias, nan):
+    """The chain over many images bit for bit its launches over up to 100 of
+    them (a workgroup an image half)."""
+    r = np.random.default_rng(300 + N)
+    x = r.uniform(0, 1, (N, C1, 32, 32)).astype(np.float32)
+    if nan:
+        x.flat[::97] = np.nan
+    w = [DevBuf.from_np((r.standard_normal(n) * 0.1).astype(np.float32))
+         for n in (32 * C1 * 9, 32, 64 * 32 * 9, 64, 4096 * 10)]
+    b1, b2 = (w[1].ptr, w[3].ptr) if bias else (None, None)
+    print("conv chain, many halves", N, C1, bias, nan, flush=True)
+
+    def run(xs, fcn):
+        n = xs.shape[0]
+        dx = DevBuf.from_np(np.ascontiguousarray(xs))
+        p1, k1 = DevBuf(n * 8192), DevBuf(n * 8192, np.uint8)
+        p2, cp, pd = DevBuf(n * 4096), DevBuf(n * 4096), DevBuf(n * 4097)
+        k2, fp = DevBuf(n * 4096, np.uint8), DevBuf(2 * n * 10)
+        sa, sb = DevBuf(32 * C1 * 9 + 32), DevBuf(18432 + 64)
+        check(tlib.tt_k_conv2d_chain_fwd(dx.ptr, w[0].ptr, b1, w[2].ptr, b2, p1.ptr, k1.ptr,
+                                         p2.ptr, cp.ptr, pd.ptr, k2.ptr, sa.ptr, sb.ptr, w[4].ptr,
+                                         fcn, fp.ptr if fcn else None, n, C1, 32, 32, 32, 64),
+              "chain")
+        out = [p1.to_np((n, 8192)), k1.to_np((n, 8192)), p2.to_np((n, 4096)),
+               cp.to_np((n, 4096)), pd.to_np((n, 4097)), k2.to_np((n, 4096))]
+        if fcn:
+            out.append(fp.to_np((2, n, 10)).transpose(1, 0, 2).copy())
+        return out, [sa.to_np((sa.n,)), sb.to_np((sb.n,))]
+
+    parts = [run(x[i:i + 100], 10) for i in range(0, N, 100)]
+    want = [np.concatenate(t) for t in zip(*[p[0] for p in parts])]
+    for fcn in (10, 0):
+        got, snap = run(x, fcn)
+        for g, e in zip(got, want):
+            assert bits_equal(g, e)
+        for g, e in zip(snap, parts[0][1]):
+            assert bits_equal(g, e)
+
+
 def test_conv_chain_rejects(tlib):
     d = DevBuf(64)
     assert tlib.tt_k_conv2d_chain_fwd(d.ptr, d.ptr, None, d.ptr, None, d.ptr, d.ptr, d.ptr, None,

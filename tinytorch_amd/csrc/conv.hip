@@ -2088,12 +2088,20 @@ constexpr int X1_SZ = 4096;
 constexpr int O_X2 = O_X1 + X1_SZ;                // pool1 slab, F1 planes
 constexpr int O_C1 = O_X2 + F1 * CS2 + 4;         // pool1 codes tile, F1 x C1T bytes
 constexpr int LDS_FLOATS = O_C1 + F1 * C1T / 4;
+constexpr int O_X1B = (LDS_FLOATS + 63) / 64 * 64;  // the other image slab (LOOP)
+constexpr int LDS_LOOP = O_X1B + X1_SZ;
+static_assert(10 * NTH <= F1 * CS2, "partial logits in the pool1 slab");
 static_assert(4 * CS1 <= X1_SZ && F2 * PT + F2 * CT / 4 <= X1_SZ, "image slab area");
 static_assert(O_X1 % 64 == 0 && O_X2 % 4 == 0 && (F1 * CS2) % 4 == 0, "alignment");
-static_assert(LDS_FLOATS * 4 <= LDS_MAX, "LDS");
+static_assert(LDS_LOOP * 4 <= LDS_MAX, "LDS");
 }  // namespace chain
 
-template <int CH2, int FCN>
+// LOOP: a workgroup per CU takes images u, u + gridDim.x, ... of nunits image
+// halves (an even grid: always the same half).  The filter banks are staged
+// once, and the next image half arrives in a second slab under phase B, so a
+// half costs its two phases and not the staging before them (1000 images: a
+// workgroup a half 146.9 us, this 125.30).  Up to 256 halves a workgroup each.
+template <int CH2, int FCN, bool LOOP>
 __global__ void __launch_bounds__(chain::NTH)
 conv_chain_fwd_kernel(const float *__restrict__ x, const float *__restrict__ w1,
                       const float *__restrict__ b1, const float *__restrict__ w2,
@@ -2102,13 +2110,14 @@ conv_chain_fwd_kernel(const float *__restrict__ x, const float *__restrict__ w1,
                       float *__restrict__ copy2, float *__restrict__ pad2,
                       unsigned char *__restrict__ codes2, float *__restrict__ snap1,
                       float *__restrict__ snap2, const float *__restrict__ fcw,
-                      float *__restrict__ fcpart, int C1) {
+                      float *__restrict__ fcpart, int C1, int nunits) {
   using namespace chain;
   extern __shared__ __attribute__((aligned(16))) float smem[];
   float *ws2 = smem + O_WS2, *ws1 = smem + O_WS1, *bs = smem + O_B;
   float *xs1 = smem + O_X1, *xs2 = smem + O_X2;
   unsigned char *c1t = (unsigned char *)(smem + O_C1);
-  const int n = blockIdx.x >> 1, hf = blockIdx.x & 1;
+  const int hf = blockIdx.x & 1;
+  int unit = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, half = lane >> 5;
@@ -2118,7 +2127,7 @@ conv_chain_fwd_kernel(const float *__restrict__ x, const float *__restrict__ w1,
   TT_PROBE(0, 0);
 
   // ---- staging: image slab, filter bank 1 (k-major), biases, then bank 2 ----
-  {
+  auto stage_image = [&](int n, float *xs) {
     const float *xn = x + (long)n * C1 * 1024;
     constexpr int T1 = 2 * CH2 * CS1;
     for (int base = wave * 256; base < T1; base += NTH * 4) {
@@ -2127,8 +2136,11 @@ conv_chain_fwd_kernel(const float *__restrict__ x, const float *__restrict__ w1,
       const int slot = rem / RS1, j = rem - slot * RS1;
       const int row = iy0 + slot;
       const bool ok = i < T1 && c < C1 && slot < R1 && j >= G1 && row >= 0 && row < 32;
-      dma_dwordx4(ok ? xn + (c * 32 + row) * 32 + (j - G1) : g_zero_src, xs1 + base);
+      dma_dwordx4(ok ? xn + (c * 32 + row) * 32 + (j - G1) : g_zero_src, xs + base);
     }
+  };
+  stage_image(unit >> 1, xs1);
+  {
     for (int base = wave * 64; base < 2 * CH2 * 9 * 32; base += NTH) {
       const int d = base + lane, k = d >> 5, f = d & 31;
       dma_dword(k < K1 ? w1 + f * K1 + k : g_zero_src, ws1 + base);
@@ -2163,12 +2175,16 @@ conv_chain_fwd_kernel(const float *__restrict__ x, const float *__restrict__ w1,
   __syncthreads();
   TT_PROBE(0, 1);
 
+  bool first = true;
+#pragma unroll 1
+  for (;;) {
+  const int n = unit >> 1;
+
   // ---- phase A: first convolution, bias, relu, pool, codes ----
   {
     const float *wa = ws1 + half * CH2 * 9 * 32 + l32;
     const float bias = bs[l32];
     const int win = l32 >> 2, dy = (l32 >> 1) & 1, dx = l32 & 1;
-    bool first = true;
     // 18 blocks (9 row pairs x 2 column halves of 8 windows), round robin
     for (int blk = wave; blk < 18; blk += 8) {
       const int i = blk >> 1, j = blk & 1;
@@ -2242,6 +2258,12 @@ conv_chain_fwd_kernel(const float *__restrict__ x, const float *__restrict__ w1,
     const unsigned *s = reinterpret_cast<const unsigned *>(c1t + f * C1T + r8 * 16);
     const uint4 v = {s[0], s[1], s[2], s[3]};
     *reinterpret_cast<uint4 *>(codes1 + ((long)n * F1 + f) * 256 + 128 * hf + 16 * r8) = v;
+  }
+
+  // the next image half, landed by the end of phase B
+  if constexpr (LOOP) {
+    const int next = unit + gridDim.x;
+    if (next < nunits) stage_image(next >> 1, xs1 == smem + O_X1 ? smem + O_X1B : smem + O_X1);
   }
 
   // the classifier rows of this thread's four pool2 features (FCN classes
@@ -2322,6 +2344,7 @@ conv_chain_fwd_kernel(const float *__restrict__ x, const float *__restrict__ w1,
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+  if constexpr (LOOP) dma_wait();  // (nothing issued since phase B began)
   __syncthreads();  // every wave is past phase A's slab: the pool2 tiles reuse it
   TT_PROBE(0, 3);
 
@@ -2376,7 +2399,8 @@ conv_chain_fwd_kernel(const float *__restrict__ x, const float *__restrict__ w1,
       // then the 512 threads' pieces of class j added in a fixed order --
       // 32 threads a class, thread l the pieces l, l + 32, ... in order (on
       // 32 banks), then a tree
-      float *red = ws2;  // the second filter bank is no longer read
+      // over the second filter bank, no longer read, or over the pool1 slab
+      float *red = LOOP ? xs2 : ws2;
 #pragma unroll
       for (int j = 0; j < FCN; j++) {
         float a = v[0] * fw[j];
@@ -2394,8 +2418,19 @@ conv_chain_fwd_kernel(const float *__restrict__ x, const float *__restrict__ w1,
       }
 #pragma unroll
       for (int m = 16; m >= 1; m >>= 1) a += __shfl_xor(a, m, 32);
-      if (j < FCN && l == 0) fcpart[((long)hf * gridDim.x / 2 + n) * FCN + j] = a;
+      if (j < FCN && l == 0) fcpart[((long)hf * (nunits >> 1) + n) * FCN + j] = a;
     }
+  }
+  if constexpr (!LOOP) break;
+  unit += gridDim.x;
+  if (unit >= nunits) break;
+  __syncthreads();  // the tiles and partial logits are read
+  if constexpr (FCN > 0) {
+    const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = tid; i < F1 * CS2 / 4; i += NTH) reinterpret_cast<f32x4 *>(xs2)[i] = z;
+    __syncthreads();
+  }
+  xs1 = xs1 == smem + O_X1 ? smem + O_X1B : smem + O_X1;
   }
   TT_PROBE(0, 4);
 }
@@ -3001,12 +3036,24 @@ extern "C" int tt_k_conv2d_chain_fwd(const float *x, const float *w1, const floa
     return -1;
   if (fail_direct()) return -3;
   if (fcpart && (fcn != 10 || !fcw)) return -1;
-  auto kern = fcpart ? (C1 > 2 ? conv_chain_fwd_kernel<2, 10> : conv_chain_fwd_kernel<1, 10>)
-                     : (C1 > 2 ? conv_chain_fwd_kernel<2, 0> : conv_chain_fwd_kernel<1, 0>);
-  constexpr size_t lds = sizeof(float) * chain::LDS_FLOATS;
+  // one workgroup a CU (its LDS); past 256 of them the same number of image
+  // halves to each, an even grid
+  const int CUS = 256, units = 2 * N, rounds = (units + CUS - 1) / CUS;
+  const bool loop = rounds > 1;
+  const int grid = loop ? ((units + rounds - 1) / rounds + 1) / 2 * 2 : units;
+  decltype(&conv_chain_fwd_kernel<1, 0, false>) kern;
+#define TT_CHAIN(FCN_)                                                                          \
+  (loop ? (C1 > 2 ? conv_chain_fwd_kernel<2, FCN_, true> : conv_chain_fwd_kernel<1, FCN_, true>) \
+        : (C1 > 2 ? conv_chain_fwd_kernel<2, FCN_, false>                                       \
+                  : conv_chain_fwd_kernel<1, FCN_, false>))
+  if (fcpart) kern = TT_CHAIN(10);
+  else kern = TT_CHAIN(0);
+#undef TT_CHAIN
+  const size_t lds = sizeof(float) * (loop ? chain::LDS_LOOP : chain::LDS_FLOATS);
   if (!allow_big_lds((const void *)kern)) return -1;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(2 * N)), dim3(chain::NTH), lds, stream(), x, w1, b1, w2,
-                     b2, pool1, codes1, pool2, copy2, pad2, codes2, snap1, snap2, fcw, fcpart, C1);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(chain::NTH), lds, stream(), x, w1, b1, w2,
+                     b2, pool1, codes1, pool2, copy2, pad2, codes2, snap1, snap2, fcw, fcpart, C1,
+                     units);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
