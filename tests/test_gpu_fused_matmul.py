@@ -582,3 +582,31 @@ def test_classifier_input_grads_taken_in_the_mlp_step(tlib):
     st.step()
     st.step(lr=0.01)
     assert tlib.tth_ce_spec_count() == n0 + 2
+
+
+# 16x16 tiles below and above a full chip: one row, part tiles, rows off 16
+# bytes (K % 4), one and two trips over K, the limits of the rule and past it
+T16_SHAPES = [(1, 784, 512), (1, 17, 33), (17, 785, 33), (16, 16, 2048), (33, 1536, 250),
+              (64, 1028, 17), (237, 1500, 260), (500, 301, 256), (250, 785, 700), (200, 512, 512),
+              (200, 513, 512), (64, 1540, 100), (1024, 1024, 256)]
+
+
+@pytest.mark.parametrize("epi", [False, True])
+@pytest.mark.parametrize("M,K,N", T16_SHAPES)
+def test_gemm_bias_t16_shapes(tlib, M, K, N, epi):
+    """C = X W + bias against float64 within (K + 1) 2^-24 of the sum of the
+    terms' magnitudes (any order of the sum), relu and pad exactly of C."""
+    X = rng.uniform(-1, 1, (M, K)).astype(np.float32)
+    W = (rng.standard_normal((K + 1, N)) / np.sqrt(K)).astype(np.float32)
+    dX, dW = DevBuf.from_np(X), DevBuf.from_np(W)
+    C, R, P = DevBuf(M * N), DevBuf(M * N), DevBuf(M * (N + 1))
+    print("gemm_bias t16", M, K, N, epi, flush=True)
+    check(tlib.tt_k_gemm_bias_relu_pad(M, N, K, dX.ptr, dW.ptr, dW.ptr + 4 * K * N, C.ptr,
+                                       R.ptr if epi else None, P.ptr if epi else None), "bias")
+    c = C.to_np((M, N))
+    x64, w64 = orc.padones_fwd(X).astype(np.float64), W.astype(np.float64)
+    bar = (K + 1) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64))
+    assert (np.abs(c - x64 @ w64) <= bar).all()
+    if epi:
+        assert bits_equal(R.to_np((M, N)), orc.relu_fwd(c))
+        assert bits_equal(P.to_np((M, N + 1)), orc.padones_fwd(orc.relu_fwd(c)))

@@ -2100,7 +2100,7 @@ static_assert(LDS_LOOP * 4 <= LDS_MAX, "LDS");
 // halves (an even grid: always the same half).  The filter banks are staged
 // once, and the next image half arrives in a second slab under phase B, so a
 // half costs its two phases and not the staging before them (1000 images: a
-// workgroup a half 146.9 us, this 125.30).  Up to 256 halves a workgroup each.
+// workgroup a half 146.9 us, this 125.3).  Up to 256 halves a workgroup each.
 template <int CH2, int FCN, bool LOOP>
 __global__ void __launch_bounds__(chain::NTH)
 conv_chain_fwd_kernel(const float *__restrict__ x, const float *__restrict__ w1,

@@ -1840,8 +1840,10 @@ gemm_small_epi_kernel(int M, int N, int K, const float *__restrict__ A, long lda
 
 // C = A * B + bias (and relu / padded relu) on 16x16 tiles for GEMMs too
 // small to fill the chip with 32x32 tiles (the MLP's hidden layers: 256 x
-// 512 x 784, 256 x 256 x 512).  A row-major M x K (rows 16-byte aligned,
-// K % 4 == 0), B row-major K x N.  Eight waves split K into equal slices of
+// 512 x 784, 256 x 256 x 512; a few samples through them).  A row-major M x K
+// (VA: rows 16-byte aligned, K % 4 == 0), B row-major K x N.  What bounds it
+// is the round trips of a launch, not the chip: one launch, no workspace and
+// no second pass.  Eight waves split K into equal slices of
 // NCH 16-k chunks; a wave issues all of its slice's loads at once (NCH x 8
 // registers a lane) so it waits for one round trip, not one per chunk, then
 // runs 4 * NCH 16x16x4 MFMAs; the wave sums are added in LDS in wave order.
@@ -1852,7 +1854,7 @@ gemm_small_epi_kernel(int M, int N, int K, const float *__restrict__ A, long lda
 // q.  Loads past the matrix are clamped to it and their values zeroed.
 typedef float f32x4t __attribute__((ext_vector_type(4)));
 constexpr int T16W = 8;  // waves per workgroup
-template <int NCH, int TN>
+template <int NCH, int TN, bool VA = true, bool LOOP = false>
 __global__ void __launch_bounds__(64 * T16W)
 gemm_t16_epi_kernel(int M, int N, int K, const float *__restrict__ A,
                     const float *__restrict__ B, SmallOut out, int kc) {
@@ -1869,34 +1871,47 @@ gemm_t16_epi_kernel(int M, int N, int K, const float *__restrict__ A,
   // after the wave sums is one more memory round trip before the stores)
   const int erow = threadIdx.x / (16 * TN), ecol = threadIdx.x % (16 * TN);
   const float bn = out.bias[min(n0 + ecol, N - 1)];
-  float4 av[NCH];
+  float av[NCH][4];
   float bv[NCH][TN][4];
-#pragma unroll
-  for (int c = 0; c < NCH; c++) {
-    const int kq = k0 + 16 * c + 4 * q;
-    av[c] = *reinterpret_cast<const float4 *>(ap + min(kq, K - 4));
-#pragma unroll
-    for (int t = 0; t < TN; t++) {
-      const float *__restrict__ bp = B + min(n0 + 16 * t + r, N - 1);
-#pragma unroll
-      for (int i = 0; i < 4; i++) bv[c][t][i] = bp[(long)min(kq + i, K - 1) * N];
-    }
-  }
   f32x4t acc[TN];
 #pragma unroll
   for (int t = 0; t < TN; t++) acc[t] = f32x4t{0.0f, 0.0f, 0.0f, 0.0f};
+  // (LOOP: a slice of several NCH chunks, NCH at a time)
+  int kp = k0;
+#pragma unroll 1
+  for (;;) {
 #pragma unroll
-  for (int c = 0; c < NCH; c++) {
-    const int kq = k0 + 16 * c + 4 * q;
-    const float a4[4] = {av[c].x, av[c].y, av[c].z, av[c].w};
+    for (int c = 0; c < NCH; c++) {
+      const int kq = kp + 16 * c + 4 * q;
+      if constexpr (VA) {
+        const float4 v = *reinterpret_cast<const float4 *>(ap + min(kq, K - 4));
+        av[c][0] = v.x; av[c][1] = v.y; av[c][2] = v.z; av[c][3] = v.w;
+      } else {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const bool in = kq + i < k1;
+        for (int i = 0; i < 4; i++) av[c][i] = ap[min(kq + i, K - 1)];
+      }
 #pragma unroll
-      for (int t = 0; t < TN; t++)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? a4[i] : 0.0f, in ? bv[c][t][i] : 0.0f,
-                                                      acc[t], 0, 0, 0);
+      for (int t = 0; t < TN; t++) {
+        const float *__restrict__ bp = B + min(n0 + 16 * t + r, N - 1);
+#pragma unroll
+        for (int i = 0; i < 4; i++) bv[c][t][i] = bp[(long)min(kq + i, K - 1) * N];
+      }
     }
+#pragma unroll
+    for (int c = 0; c < NCH; c++) {
+      const int kq = kp + 16 * c + 4 * q;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const bool in = kq + i < k1;
+#pragma unroll
+        for (int t = 0; t < TN; t++)
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? av[c][i] : 0.0f, in ? bv[c][t][i] : 0.0f,
+                                                        acc[t], 0, 0, 0);
+      }
+    }
+    if constexpr (!LOOP) break;
+    kp += 16 * NCH;
+    if (kp >= k1) break;
   }
   // every wave's sums to LDS; then each thread adds the eight wave sums of
   // its output in wave order and stores it (the stores spread over the
@@ -1988,39 +2003,44 @@ gemm_t16_split_kernel(int M, int N, int K, const float *__restrict__ A, long lda
 }
 
 // The 16x16-tile forward when it applies: 0 launched, 1 not covered, < 0
-// launch error.  Taken for at least 256 tiles (one a CU) and at most 1024,
-// K <= 1024.
+// launch error.  Few enough tiles that all of them are on the chip at once (four
+// workgroups a CU at most) and a k slice that a wave loads in one or two round
+// trips.  Measured against the split-K kernel and its reduction, us a call:
+// 1 x 784 x 512 4.7 / 8.1, 64 x 784 x 256 5.1 / 8.2, 237 x 784 x 260 5.4 /
+// 11.2, 250 x 784 x 700 9.0 / 15.2; K = 1500 64 x 256 6.8 / 9.2, but at 416
+// tiles 10.9 / 11.4 and K = 3072 64 x 256 11.3 / 10.5, so a second trip up to
+// K = 1536 and 256 tiles.  A with rows off 16 bytes is loaded an element a
+// lane: 16 x 785 x 512 7.4 / 8.7, 250 x 785 x 700 12.6 / 15.5, but K = 1501
+// 10.9 / 9.2, and 256 to 512 tiles (two workgroups of 16 columns on some CUs)
+// 301 6.5 / 8.7, 785 12.3 / 10.6.
 int run_t16(int M, int N, int K, const float *A, const float *B, const SmallOut &out) {
   const long tiles = (long)((M + 15) / 16) * ((N + 15) / 16);
-  if (!g_t16 || K < 16 || K % 4 || !aligned16(A) || tiles < 256 || tiles > 1024 ||
-      K > 1024 || (M + 15) / 16 > 65535)
-    return 1;
-  static_assert(T16W == 8, "K <= 1024 is at most 8 chunks of 16 k a wave");
-  const int nch = (K + 16 * T16W - 1) / (16 * T16W);  // 16-k chunks a wave
-  const int kc = 16 * nch;
+  const bool va = aligned16(A) && K % 4 == 0;
+  const int kmax = va ? (tiles <= 256 ? 1536 : 1024) : tiles <= 256 || tiles >= 512 ? 1024 : 512;
+  if (!g_t16 || K < 16 || tiles > 1024 || K > kmax || (M + 15) / 16 > 65535) return 1;
+  const int chunks = (K + 16 * T16W - 1) / (16 * T16W);  // 16-k chunks a wave
+  const int passes = (chunks + 7) / 8, nch = (chunks + passes - 1) / passes;
+  const int kc = 16 * nch * passes;
   // two column blocks a workgroup (16x32 tiles, each A fragment feeding two
   // MFMAs) while that still leaves 256 workgroups (the MLP's 256x512x784:
   // step 0.0463 -> 0.0453 ms); at 256 tiles the halved grid is slower
   const int tn = tiles >= 512 ? 2 : 1;
   const dim3 grid((unsigned)((N + 16 * tn - 1) / (16 * tn)), (unsigned)((M + 15) / 16));
-#define TT_T16(NCH_)                                                                          \
-  if (tn == 2)                                                                                \
-    hipLaunchKernelGGL((gemm_t16_epi_kernel<NCH_, 2>), grid, dim3(64 * T16W), 0, stream(), M, N, \
-                       K, A, B, out, kc);                                                     \
-  else                                                                                        \
-    hipLaunchKernelGGL((gemm_t16_epi_kernel<NCH_, 1>), grid, dim3(64 * T16W), 0, stream(), M, N, \
-                       K, A, B, out, kc)
-  switch (nch) {
-    case 1: TT_T16(1); break;
-    case 2: TT_T16(2); break;
-    case 3: TT_T16(3); break;
-    case 4: TT_T16(4); break;
-    case 5: TT_T16(5); break;
-    case 6: TT_T16(6); break;
-    case 7: TT_T16(7); break;
-    default: TT_T16(8); break;  // K <= 1024: at most 8 chunks a wave
-  }
+  decltype(&gemm_t16_epi_kernel<1, 1>) kern = nullptr;
+#define TT_T16(NCH_)                                                                       \
+  case NCH_:                                                                               \
+    if (passes > 1) {                                                                      \
+      if constexpr (NCH_ == 5 || NCH_ == 6) kern = gemm_t16_epi_kernel<NCH_, 1, true, true>; \
+    } else if (tn == 2) {                                                                  \
+      kern = va ? gemm_t16_epi_kernel<NCH_, 2> : gemm_t16_epi_kernel<NCH_, 2, false>;      \
+    } else {                                                                               \
+      kern = va ? gemm_t16_epi_kernel<NCH_, 1> : gemm_t16_epi_kernel<NCH_, 1, false>;      \
+    }                                                                                      \
+    break;
+  switch (nch) { TT_T16(1) TT_T16(2) TT_T16(3) TT_T16(4) TT_T16(5) TT_T16(6) TT_T16(7) TT_T16(8) }
 #undef TT_T16
+  if (!kern) return 1;
+  hipLaunchKernelGGL(kern, grid, dim3(64 * T16W), 0, stream(), M, N, K, A, B, out, kc);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
