@@ -120,8 +120,8 @@ int tth_gemm_mid_force(int on);
 int tth_gemm_small(int on);
 /* Tuning hook: 0 disables, 1 (default) enables the 16x16-tile kernels (K
  * split over eight waves, each loading its whole slice before its MFMAs):
- * tt_k_gemm_bias_relu_pad's for 256-1024 output tiles of 16x16, K <= 1024,
- * 16-byte aligned A rows; and the split-K partials of GEMMs with N <= 16
+ * tt_k_gemm_bias_relu_pad's for up to 1024 output tiles of 16x16, K <= 1024 or 1536,
+ * shorter for rows of A that are not 16-byte aligned; and the split-K partials of GEMMs with N <= 16
  * and K >= 2048 (at most 128 tiles). */
 int tth_gemm_t16(int on);
 /* Diagnostics: how many classifier backward rules took the input gradients
@@ -172,8 +172,9 @@ int tt_k_softmax_bwd(const float *s, const float *g, float *dx, long rows, int c
  * reference tests/gate_cifar_cnn.py:175-181 on the device. */
 int tt_k_softmax_ce(const float *logits, const int32_t *labels, float *probs,
                     float *loss_rows, float *seed, long rows, int cols, float scale);
-/* Same, for rows <= TT_CE_MEAN_MAX_ROWS, in one launch that also reduces the
- * mean loss into loss_mean[0] (fixed reduction order). */
+/* Same, for rows <= TT_CE_MEAN_MAX_ROWS, that also reduces the mean loss into
+ * loss_mean[0] (fixed reduction order): one launch up to 256 rows and 32
+ * columns, a launch over the rows and one over their losses above. */
 #define TT_CE_MEAN_MAX_ROWS 8192
 int tt_k_softmax_ce_mean(const float *logits, const int32_t *labels, float *probs,
                          float *loss_mean, float *seed, long rows, int cols, float scale);

@@ -2230,8 +2230,9 @@ int run_ring(int splits, int kc, int M, int N, int K, const Opnd &A, const Opnd 
 // Estimated microseconds of each kernel on one block of C: whole rounds of
 // 256 CUs times a tile's K loop, at the per-k times measured (us a round and
 // k: 64x64 tiles 0.0185 alone on a CU, 0.040 two a CU and 0.018 for a last
-// half round (2048 x 1024 x 1024 39.3 us, 709 x 3052 x 1617 93); 128x128 0.064 (2048^3 136 us, 126 TFLOP/s, where register-staged
-// tiles took 155); 256x64 0.075; 256x256 0.2265; 4-byte loads 8-16 % more).
+// half round (2048 x 1024 x 1024 39.3 us, 709 x 3052 x 1617 93); 128x128 0.064
+// (2048^3 136 us, 126 TFLOP/s, where register-staged tiles took 155); 256x64
+// 0.075; 256x256 0.2265; 4-byte loads 8-16 % more).
 // A grid a little over a round costs a whole one more, so the rows or columns
 // past the last full round may run as a GEMM of their own (4097 x 4095 x 4093:
 // 2541 us on 256x128 register-staged tiles; 1416 as one grid of 33 x 32 tiles;
