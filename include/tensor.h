@@ -34,6 +34,7 @@ typedef struct Tensor {
     /* ---- appended: not part of the reference layout ---- */
     float *dev;      /* device payload, numel floats */
     int    valid;    /* bit 0: device copy current, bit 1: host copy current */
+    unsigned writes; /* times it was handed to the host (tt_data) or changed in place */
 } Tensor;
 
 /* lifecycle -- reference include/tensor.h:20-23, src/tensor.c:10-61 */

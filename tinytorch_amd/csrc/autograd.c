@@ -52,6 +52,8 @@ struct AGNode {
         struct { int kh, kw, sh, sw; Tensor *codes; } win;  /* pools (codes: one byte a
                                                       2x2 window, or NULL) */
         struct { int sh, sw, ph, pw; float *col; int col_ones; } conv;
+        struct { unsigned src, own; } pad;  /* padones: the writes of its input and of its
+                                               value when it was made (padones_input) */
         /* softmax-CE; sda: the input gradients of its classifier (see
          * ce_spec), computed with the seed and not yet handed over */
         struct { Tensor *probs, *seed; int32_t *labels; Tensor *sda[3]; int *stale; } ce;
@@ -275,10 +277,14 @@ AGNode *ag_mulscalar(AGNode *a, float s) {
 
 /* The input of a padones node, when a is one: a matmul of a padones output
  * [X, 1] * W is X * W[:K-1] + W[K-1] (the weights' last row added to every
- * row), computed from X's aligned rows without reading the ones column. */
+ * row), computed from X's aligned rows without reading the ones column.  Only
+ * while the two agree: the node's value is X as it was when the node was made,
+ * whatever is written to X later (by the host, or a step of a leaf), and the
+ * host may write the value itself. */
 static const Tensor *padones_input(const AGNode *a) {
     if (a->op != &OP_PADONES || !a->in[0]) return NULL;
     const Tensor *x = a->in[0]->val;
+    if (x->writes != a->at.pad.src || a->val->writes != a->at.pad.own) return NULL;
     return x && x->ndim == 2 && x->shape[1] >= 1 && a->val->shape[1] == x->shape[1] + 1 ? x
                                                                                        : NULL;
 }
@@ -398,6 +404,15 @@ AGNode *ag_softmax(AGNode *a) {
     return make_node(tt_softmax(a->val), &OP_SOFTMAX, a, NULL, NULL);
 }
 
+static AGNode *padones_node(Tensor *v, AGNode *a) {
+    AGNode *n = make_node(v, &OP_PADONES, a, NULL, NULL);
+    if (n) {
+        n->at.pad.src = a->val->writes;
+        n->at.pad.own = n->val->writes;
+    }
+    return n;
+}
+
 AGNode *ag_padones(AGNode *a) {
     if (!a || a->val->ndim != 2) return NULL;
     const long M = a->val->shape[0], K = a->val->shape[1];
@@ -409,7 +424,7 @@ AGNode *ag_padones(AGNode *a) {
          * softmax-CE can join it */
         Tensor *v = tt_chain_ready() ? tt_empty_dev(shp, 2) : NULL;
         if (v) {
-            AGNode *n = make_node(v, &OP_PADONES, a, NULL, NULL);
+            AGNode *n = padones_node(v, a);
             if (n) {
                 tt_pend.d = v;
                 tt_pend.active = TT_PEND_CHAIN_PAD;
@@ -437,7 +452,7 @@ AGNode *ag_padones(AGNode *a) {
                 if (tt_lazy_relu(p.r, p.out) != 0 &&
                     tt_k_relu_fwd(p.out->dev, p.r->dev, p.r->numel) != 0)
                     p.r->valid = 0;
-                return make_node(v, &OP_PADONES, a, NULL, NULL);
+                return padones_node(v, a);
             }
             tt_pend = p;  /* not launched: the chain runs below, then the padones */
             tt_release(v);
@@ -451,7 +466,7 @@ AGNode *ag_padones(AGNode *a) {
             const TTPendConv p = tt_pend;
             tt_pend.active = 0;
             if (tt_k_copy_padones_fwd(p.x, p.out->dev, v->dev, M, K) == 0)
-                return make_node(v, &OP_PADONES, a, NULL, NULL);
+                return padones_node(v, a);
             tt_pend = p;  /* not launched: the plain copy runs below */
             tt_release(v);
         }
@@ -466,12 +481,12 @@ AGNode *ag_padones(AGNode *a) {
                 ttk_gemm_bias_relu(p.geo[0], p.geo[1], p.geo[2], p.x, p.w, p.b, p.out->dev,
                                    p.r->dev) == 0 &&
                 (tt_lazy_padones(v, a->val) == 0 || tt_k_padones_fwd(p.r->dev, v->dev, M, K) == 0))
-                return make_node(v, &OP_PADONES, a, NULL, NULL);
+                return padones_node(v, a);
             if ((p.b ? tt_k_gemm_bias_relu_pad(p.geo[0], p.geo[1], p.geo[2], p.x, p.w, p.b,
                                                p.out->dev, p.r->dev, v->dev)
                      : tt_k_gemm_relu_pad(p.geo[0], p.geo[1], p.geo[2], p.x, p.w, p.out->dev,
                                           p.r->dev, v->dev)) == 0)
-                return make_node(v, &OP_PADONES, a, NULL, NULL);
+                return padones_node(v, a);
             tt_pend = p;  /* not launched: the plain matmul and relu run below */
             tt_release(v);
         }
@@ -482,7 +497,7 @@ AGNode *ag_padones(AGNode *a) {
             const TTPendConv p = tt_pend;
             tt_pend.active = 0;
             if (tt_k_relu_padones_fwd(p.x, p.out->dev, v->dev, M, K) == 0)
-                return make_node(v, &OP_PADONES, a, NULL, NULL);
+                return padones_node(v, a);
             tt_pend = p;  /* not launched: the plain relu runs below */
             tt_release(v);
         }
@@ -500,7 +515,7 @@ AGNode *ag_padones(AGNode *a) {
         tt_release(v);
         return NULL;
     }
-    return make_node(v, &OP_PADONES, a, NULL, NULL);
+    return padones_node(v, a);
 }
 
 AGNode *ag_reshape(AGNode *a, const long *new_shape, int new_ndim) {
@@ -907,7 +922,7 @@ static int backward_matmul_spec(AGNode *n) {
     AGNode *a = n->in[0], *b = n->in[1];
     AGNode *x = a->in[0];
     const int M = (int)a->val->shape[0], K = (int)a->val->shape[1], N = (int)b->val->shape[1];
-    const int ok = !stale && n->fanin == 1 && a->op == &OP_PADONES && a->fanin == 1 && !a->grad &&
+    const int ok = !stale && n->fanin == 1 && padones_input(a) && a->fanin == 1 && !a->grad &&
                    relu_fusable(x) && !x->grad && needs(b) && tt_defer_enabled() &&
                    ttk_gemm_tn_padones_any(M, K - 1, N, NULL, NULL, NULL) == 0;
     Tensor *gb = ok ? tt_empty_like(b->val) : NULL;
@@ -949,7 +964,7 @@ static void backward_matmul(AGNode *n) {
     const float *g = tt_dev(n->grad);
     if (!g) return;
     if (tt_defer_enabled() && backward_matmul_fused(n, g, NULL) == 0) return;
-    if (needs(b) && !needs(a) && a->op == &OP_PADONES && K > 1) {
+    if (needs(b) && !needs(a) && padones_input(a) && K > 1) {
         /* dB from the padones input: the padded copy is not read; with the
          * deferral, dB is a recipe that the optimizer's step runs in its own
          * launch (or the first read runs by itself) */
@@ -976,11 +991,11 @@ static void backward_matmul(AGNode *n) {
         if (ga && tt_k_gemm(M, K, N, g, N, 0, bd, N, 1, ga->dev, K) == 0) accum_move(a, ga);
         else tt_release(ga);
     }
-    /* (a padded value that the host holds may have been changed there) */
-    const Tensor *xp = needs(b) && K > 1 && pad_unwritten(M, K - 1) && a->val->valid & TT_V_DEV
+    const Tensor *xp = needs(b) && K > 1 && pad_unwritten(M, K - 1) &&
+                               tt_lazy_padones_pending(a->val)
                            ? padones_input(a)
                            : NULL;
-    if (xp) {  /* dB from the padones input */
+    if (xp) {  /* dB from the padones input: the padded value was never written */
         const float *xd = tt_dev((Tensor *)xp);
         Tensor *gb = xd ? tt_empty_like(b->val) : NULL;
         if (gb && ttk_gemm_tn_colsum(M, K - 1, N, xd, g, gb->dev) == 0) accum_move(b, gb);

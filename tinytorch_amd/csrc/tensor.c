@@ -565,6 +565,13 @@ restart:
 
 void tt_lazy_before_write(Tensor *t) {
     if (g_lazy_vals && t) lazy_take(t, 1, 0);
+    if (t) t->writes++;
+}
+
+int tt_lazy_padones_pending(const Tensor *t) {
+    for (TTLazyVal *l = g_lazy_vals; l; l = l->next)
+        if (l->t == t && l->kind == 1) return 1;
+    return 0;
 }
 
 void tt_release(Tensor *t) {
@@ -597,6 +604,7 @@ float *tt_data(const Tensor *ct) {
         lazy_take(t, 1, 0);  /* the host may write t: recipes reading it run now */
     }
     if (!t || !t->valid) return NULL;
+    t->writes++;
     if (!(t->valid & TT_V_HOST)) {
         if (!t->data) {
             t->data = (float *)ttrt_host_alloc(sizeof(float) * (size_t)t->numel);

@@ -123,8 +123,12 @@ int tt_lazy_ce_job(Tensor *const out[4], Tensor *w, float *ws, const float *bias
  * otherwise.  tt_lazy_ce_done(job): a kernel wrote the job's outputs */
 int tt_lazy_ce_args(const Tensor *t, TTHeadCeArgs *a, void **job);
 void tt_lazy_ce_done(void *job);
-/* t is about to be changed in place: run the recipes that read it */
+/* t is about to be changed in place: run the recipes that read it and count
+ * the write */
 void tt_lazy_before_write(Tensor *t);
+/* t is a padones recipe no access has run: the source's device copy is still
+ * the one it was made from */
+int tt_lazy_padones_pending(const Tensor *t);
 Tensor *tt_lazy_relu_src(const Tensor *t);  /* src while t is still unwritten */
 int tt_defer_enabled(void);
 Tensor *tt_reshape_ex(const Tensor *a, const long *new_shape, int new_ndim, int defer);
