@@ -43,7 +43,7 @@ def test_softmax_ce_rows(tlib, rows, cols):
     # the sum, the division), stays as 2.4e-7 of the seed's scale
     np.testing.assert_allclose(X.grad(), s64, rtol=1e-5, atol=4e-7 / rows)
     np.testing.assert_allclose(loss.value(), [l64.mean()], rtol=1e-5)
-    loss.backward(None)  # recomputed from the kept labels and added
+    loss.backward(None)  # the kept seed, added
     np.testing.assert_allclose(X.grad(), 2 * s64, rtol=1e-5, atol=8e-7 / rows)
     # the device entry, its mean added in the order of the row losses
     dx, dl = DevBuf.from_np(x), DevBuf.from_np(y)
@@ -72,3 +72,35 @@ def test_softmax_small_rows(tlib):
         keep = np.arange(rows) != rows // 2
         e = np.exp(x[keep].astype(np.float64) - x[keep].max(1, keepdims=True, initial=-1e30))
         np.testing.assert_allclose(got[keep], e / e.sum(1, keepdims=True), rtol=1e-5)
+
+
+@pytest.mark.parametrize("rows,cols", [(40, 10), (513, 10), (700, 70)])
+@pytest.mark.parametrize("what", ["logits", "gradient", "stepped"])
+def test_second_backward_has_the_forward_seed(tlib, rows, cols, what):
+    """Between two backward passes the host writes the logits or their
+    gradient, or a step changes them in place: the second pass still gives the
+    forward's seed (fp32: the bounds of test_softmax_ce_rows)."""
+    from tinytorch_amd.torch_py import LIB, Node
+    rng = np.random.default_rng(rows + cols)
+    x = (rng.standard_normal((rows, cols)) * 3).astype(np.float32)
+    y = rng.integers(0, cols, rows).astype(np.int32)
+    s64 = _ref(x, y)[1]
+    X = Node.leaf(x)
+    loss = X.softmax_ce(y)
+    loss.backward(None)
+    n = rows * cols
+    if what == "logits":
+        np.ctypeslib.as_array(LIB.tt_data(LIB.ag_value(X.ptr)), shape=(n,))[:] = 1
+    elif what == "stepped":
+        X.sgd_step(1e3)
+    else:
+        np.ctypeslib.as_array(LIB.tt_data(LIB.ag_grad(X.ptr)), shape=(n,))[:] = 5
+    loss.backward(None)
+    first = 5.0 if what == "gradient" else s64
+    np.testing.assert_allclose(X.grad(), first + s64, rtol=1e-5,
+                               atol=4e-7 if what == "gradient" else 8e-7 / rows)
+    loss.backward(None)
+    np.testing.assert_allclose(X.grad(), first + 2 * s64, rtol=1e-5,
+                               atol=8e-7 if what == "gradient" else 1.2e-6 / rows)
+    for node in (loss, X):
+        node.release()

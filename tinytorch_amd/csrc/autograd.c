@@ -56,7 +56,7 @@ struct AGNode {
                                                value when it was made (padones_input) */
         /* softmax-CE; sda: the input gradients of its classifier (see
          * ce_spec), computed with the seed and not yet handed over */
-        struct { Tensor *probs, *seed; int32_t *labels; Tensor *sda[3]; int *stale; } ce;
+        struct { Tensor *probs, *seed; Tensor *sda[3]; int *stale; } ce;
         /* matmul: sda handed over by its softmax-CE; *stale set when the
          * weights they were formed with are about to change */
         struct { Tensor *sda[3]; int *stale; } mm;
@@ -110,7 +110,6 @@ static void spec_drop(Tensor *sda[3], int **stale) {
 static void drop_ce(AGNode *n) {
     tt_release(n->at.ce.probs);
     tt_release(n->at.ce.seed);
-    free(n->at.ce.labels);
     spec_drop(n->at.ce.sda, &n->at.ce.stale);
 }
 static void drop_mm(AGNode *n) { spec_drop(n->at.mm.sda, &n->at.mm.stale); }
@@ -686,11 +685,11 @@ AGNode *ag_softmax_ce(AGNode *logits, const int *labels, long rows) {
             if (rc == 0 && (tt_lazy_ce_mean(loss, rl) == 0 ||
                             tt_k_ce_mean_rows(tt_dev(rl), loss->dev, (int)rows) == 0)) {
                 tt_release(rl);
+                free(hlab);
                 AGNode *n = make_node(loss, &OP_SOFTMAX_CE, logits, NULL, NULL);
-                if (!n) { tt_release(probs); tt_release(seed); free(hlab); return NULL; }
+                if (!n) { tt_release(probs); tt_release(seed); return NULL; }
                 n->at.ce.probs = probs;
                 n->at.ce.seed = seed;
-                n->at.ce.labels = hlab;
                 return n;
             }
             /* the reduction did not run: the logits from the GEMM (the
@@ -721,15 +720,15 @@ AGNode *ag_softmax_ce(AGNode *logits, const int *labels, long rows) {
         if (rc == 0 && (tt_lazy_ce_mean(loss, rl) == 0 ||
                         tt_k_ce_mean_rows(rl->dev, loss->dev, (int)rows) == 0)) {
             tt_release(rl);
+            free(hlab);
             AGNode *n = make_node(loss, &OP_SOFTMAX_CE, logits, NULL, NULL);
             if (!n) {
-                tt_release(probs); tt_release(seed); free(hlab);
+                tt_release(probs); tt_release(seed);
                 spec_drop(sda, &stale);
                 return NULL;
             }
             n->at.ce.probs = probs;
             n->at.ce.seed = seed;
-            n->at.ce.labels = hlab;
             for (int i = 0; i < 3; i++) n->at.ce.sda[i] = sda[i];
             n->at.ce.stale = stale;
             return n;
@@ -753,15 +752,15 @@ AGNode *ag_softmax_ce(AGNode *logits, const int *labels, long rows) {
                    (tt_lazy_ce_mean(loss, rl) == 0 ||
                     tt_k_ce_mean_rows(rl->dev, loss->dev, (int)rows) == 0);
     tt_release(rl);
+    free(hlab);
     if (!ok) {
-        tt_release(probs); tt_release(seed); tt_release(loss); free(hlab);
+        tt_release(probs); tt_release(seed); tt_release(loss);
         return NULL;
     }
     AGNode *n = make_node(loss, &OP_SOFTMAX_CE, logits, NULL, NULL);
-    if (!n) { tt_release(probs); tt_release(seed); free(hlab); return NULL; }
+    if (!n) { tt_release(probs); tt_release(seed); return NULL; }
     n->at.ce.probs = probs;
     n->at.ce.seed = seed;
-    n->at.ce.labels = hlab;
     return n;
 }
 
@@ -1455,29 +1454,18 @@ static int is_host_one(const Tensor *t) {
 }
 
 /* d logits = seed * dL (dL is the 1-element incoming gradient).  With dL
- * exactly 1 the product is the seed itself: the first backward moves the
- * seed tensor into the logits' gradient (no kernel); a later one recomputes
- * it (same kernel, same inputs, same bits) from the kept host labels. */
+ * exactly 1 the product is the seed itself: the seed tensor becomes the
+ * logits' gradient (no kernel), and a recipe of its copy, run only when that
+ * gradient is about to be written or a later backward reads it, is kept in its
+ * place -- the seed of the forward whatever has happened to the logits. */
 static void backward_softmax_ce(AGNode *n) {
     AGNode *a = n->in[0];
-    if (!needs(a)) return;
-    if (!n->at.ce.seed && n->at.ce.labels) {
-        const float *x = tt_dev(a->val);
-        const long rows = a->val->shape[0];
-        const int cols = (int)a->val->shape[1];
-        Tensor *p = tt_empty_like(a->val), *s = tt_empty_like(a->val);
-        const int ok = x && p && s &&
-                       ttk_ce_rows(x, n->at.ce.labels, p->dev, s->dev, NULL, rows, cols,
-                                   1.0f / (float)rows) == 0;
-        tt_release(p);
-        if (!ok) { tt_release(s); return; }
-        n->at.ce.seed = s;
-    }
-    if (!n->at.ce.seed) return;
+    if (!needs(a) || !n->at.ce.seed) return;
     if (is_host_one(n->grad)) {
-        if (n->at.ce.labels && !a->grad) {
-            a->grad = n->at.ce.seed;
-            n->at.ce.seed = NULL;
+        Tensor *seed = n->at.ce.seed, *kept = a->grad ? NULL : tt_empty_like(seed);
+        if (kept && tt_lazy_copy(kept, seed) == 0) {
+            a->grad = seed;
+            n->at.ce.seed = kept;
             if (n->at.ce.sda[0] && a->op == &OP_MATMUL && !a->at.mm.sda[0]) {
                 /* the seed is the logits' gradient as it stands: the
                  * classifier's input gradients formed with it go along */
@@ -1489,7 +1477,8 @@ static void backward_softmax_ce(AGNode *n) {
                 n->at.ce.stale = NULL;
             }
         } else {
-            accum_copy(a, n->at.ce.seed);
+            tt_release(kept);
+            accum_copy(a, seed);
         }
         return;
     }

@@ -137,7 +137,8 @@ typedef struct TTLazyVal {
                                   two-convolution chain did not store; 6: see
                                   ce (every output is written at once); 7:
                                   src without its last column (padones
-                                  backward, dims M K); 8: a guard (flag) */
+                                  backward, dims M K); 8: a guard (flag); 9: a copy
+                                  of src */
     TTDwtShared *dwt;
     Tensor *src2;
     int dims[3];
@@ -170,6 +171,7 @@ static int lazy_add(Tensor *t, Tensor *src, int kind) {
 int tt_lazy_relu(Tensor *t, Tensor *src) { return lazy_add(t, src, 0); }
 int tt_lazy_padones(Tensor *t, Tensor *src) { return lazy_add(t, src, 1); }
 int tt_lazy_ce_mean(Tensor *t, Tensor *src) { return lazy_add(t, src, 2); }
+int tt_lazy_copy(Tensor *t, Tensor *src) { return lazy_add(t, src, 9); }
 int tt_lazy_guard(Tensor *src, int *flag) {
     if (lazy_add(NULL, src, 8) != 0) return -1;
     g_lazy_vals->flag = flag;
@@ -547,6 +549,7 @@ restart:
                            : l->kind == 4 ? ttk_gemm_tn_padones_any(l->dims[0], l->dims[1],
                                                                     l->dims[2], x, x2, l->t->dev)
                            : l->kind == 7 ? tt_k_padones_bwd(x, l->t->dev, l->dims[0], l->dims[1])
+                           : l->kind == 9 ? tt_k_copy(l->t->dev, x, l->t->numel)
                            : l->kind == 5 ? tt_conv_fwd_any(x, l->buf,
                                                             l->buf + (long)l->q[4] * l->q[1] *
                                                                          l->q[5] * l->q[6],

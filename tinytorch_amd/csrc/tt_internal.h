@@ -90,6 +90,7 @@ int tt_lazy_conv(Tensor *t, Tensor *x, float *snap, const int *q);
 int tt_lazy_relu(Tensor *t, Tensor *src);
 int tt_lazy_padones(Tensor *t, Tensor *src);  /* t (M x K+1) = padones(src (M x K)) */
 int tt_lazy_ce_mean(Tensor *t, Tensor *src);  /* t (1) = mean of the row losses src */
+int tt_lazy_copy(Tensor *t, Tensor *src);  /* t = src as it is now */
 /* dw, db (db may be NULL) = the pending reduction job; 0 ok, -1 (no memory):
  * run the job now */
 int tt_lazy_dwt(Tensor *dw, Tensor *db, const TTDwtJob *job);
