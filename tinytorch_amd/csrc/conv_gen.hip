@@ -255,6 +255,7 @@ struct ConvG {
   int F, OH, OW;       // the output (dX: the input gradient)
   int HH, WW, sh, sw, ph, pw;
   int ck, cs, lda;     // channels a chunk, floats a slab channel, A's row stride (largest)
+  int close;           // quads a wave sums in one chain
   int ftiles;
 };
 
@@ -288,6 +289,38 @@ __device__ __forceinline__ void mul_quad(float (*a)[4], float (*b)[4], f32x16 (*
 #pragma unroll
       for (int j = 0; j < NJ; j++)
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][s], b[j][s], acc[i][j], 0, 0, 0);
+}
+
+template <int MI, int NJ>
+__device__ __forceinline__ void clear(f32x16 (&a)[MI][NJ]) {
+#pragma unroll
+  for (int i = 0; i < MI; i++)
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+      for (int q = 0; q < 16; q++) a[i][j][q] = 0.f;
+}
+
+// The products of a few quads are summed by themselves and then added to the
+// tile's sums: a chain of all of them rounds as often as it is long.  Relative
+// error against 64 bits in one chain, closed as now, and of the GEMM that ran
+// these before:
+//   forward, a chunk a chain: 32 x 64 x 56 x 56 -> 128 4.3e-7, 1.6e-7, 4.3e-7
+//     (145 -> 150 us); 2 x 115 x 10 x 27 -> 28, 5 x 5, stride 2: 4.5e-7,
+//     1.5e-7, 1.8e-7
+//   dX, 32 x 64 x 56 x 56 -> 128: 6.0e-7, 1.7e-7, 2.1e-7 (167 -> 172 us); few
+//     filters, whose GEMM summed few products a tap, close every 32 products:
+//     50 x 24 x 45 x 37 -> 40, 5 x 5, stride 2: 2.9e-7, 1.2e-7, 1.3e-7 (31 ->
+//     32 us)
+//   dW, 32 pixels a chain: 4.8e-7, 1.6e-7, 9.9e-7 and 2.6e-7, 1.4e-7, 3.3e-7
+template <int MI, int NJ>
+__device__ __forceinline__ void add(f32x16 (&a)[MI][NJ], const f32x16 (&b)[MI][NJ]) {
+#pragma unroll
+  for (int i = 0; i < MI; i++)
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+      for (int q = 0; q < 16; q++) a[i][j][q] += b[i][j][q];
 }
 
 // Forward (DX false) and input gradient (DX true).  Waves: WM x WN of them
@@ -428,12 +461,7 @@ conv_gen_kernel(const ConvG g) {
   }
 
   f32x16 acc[MI][NJ];
-#pragma unroll
-  for (int i = 0; i < MI; i++)
-#pragma unroll
-    for (int j = 0; j < NJ; j++)
-#pragma unroll
-      for (int q = 0; q < 16; q++) acc[i][j][q] = 0.f;
+  clear(acc);
 
   auto multiply = [&](int ch) {
     const float *const as = smem;
@@ -441,10 +469,16 @@ conv_gen_kernel(const ConvG g) {
     const int kh = (min(g.ck, g.C - ch * g.ck) * T + 7) / 8 * 4;  // indices a lane half
     const float *const al = as + (wm * MI * 32 + l32) * lda + h * kh;
     const int *const tl = tab + h * kh;
-    for (int q = 4 * wk; q < kh; q += 4 * KW) {
-      float a[MI][4], bb[NJ][4];
-      read_quad<MI, NJ>(a, bb, al + q, 32 * lda, xs, pix, tl + q);
-      mul_quad<MI, NJ>(a, bb, acc);
+    for (int q = 4 * wk; q < kh;) {
+      const int end = min(kh, q + 4 * KW * g.close);
+      f32x16 part[MI][NJ];
+      clear(part);
+      for (; q < end; q += 4 * KW) {
+        float a[MI][4], bb[NJ][4];
+        read_quad<MI, NJ>(a, bb, al + q, 32 * lda, xs, pix, tl + q);
+        mul_quad<MI, NJ>(a, bb, part);
+      }
+      add(acc, part);
     }
   };
 
@@ -635,15 +669,10 @@ conv_gen_dw_kernel(const ConvGW g) {
   }
 
   f32x16 acc[MI][NJ];
+  clear(acc);
   float sum[MI];
 #pragma unroll
-  for (int i = 0; i < MI; i++) {
-    sum[i] = 0.f;
-#pragma unroll
-    for (int j = 0; j < NJ; j++)
-#pragma unroll
-      for (int q = 0; q < 16; q++) acc[i][j][q] = 0.f;
-  }
+  for (int i = 0; i < MI; i++) sum[i] = 0.f;
   const bool want_db = g.db && ct == 0 && wn == 0;
 
   auto multiply = [&](int ch) {
@@ -653,7 +682,7 @@ conv_gen_dw_kernel(const ConvGW g) {
     const int kh = (np + 7) / 8 * 4;
     const float *const al = smem + (wm * MI * 32 + l32) * PC;
     const int *const tl = tab + h * kh;
-    auto quad = [&](int q, bool edge) {
+    auto quad = [&](int q, bool edge, f32x16 (&acc)[MI][NJ]) {
       float a[MI][4], bb[NJ][4];
       read_quad<MI, NJ>(a, bb, al + 4 * (((h * kh + q) >> 2) ^ (l32 & 15)), 32 * PC, xs, ko, tl + q);
       if (edge) {  // pixels past the range: zeros in both operands
@@ -672,10 +701,16 @@ conv_gen_dw_kernel(const ConvGW g) {
       }
       mul_quad<MI, NJ>(a, bb, acc);
     };
-    if (np == PC)
-      for (int q = 0; q < PC / 2; q += 4) quad(q, false);
-    else
-      for (int q = 0; q < kh; q += 4) quad(q, true);
+    if (np == PC) {
+      for (int q0 = 0; q0 < PC / 2; q0 += PC / 4) {
+        f32x16 part[MI][NJ];
+        clear(part);
+        for (int q = q0; q < q0 + PC / 4; q += 4) quad(q, false, part);
+        add(acc, part);
+      }
+    } else {
+      for (int q = 0; q < kh; q += 4) quad(q, true, acc);
+    }
   };
 
   zero_lds(smem + asz, slab_sz, tid);  // the padding columns, which no load writes
@@ -712,7 +747,8 @@ conv_gen_dw_kernel(const ConvGW g) {
 }
 
 // dw, db = the sum of Z partials of F rows of K + 1 (the last column db's) in
-// order: 64 outputs a workgroup, the splits dealt to its four waves.
+// a fixed order: 64 outputs a workgroup, the splits dealt to its four waves,
+// four chains each.
 __global__ void __launch_bounds__(NT) conv_gen_dw_reduce(const float *__restrict__ part, float *dw,
                                                          float *db, int Z, int F, int K) {
   __shared__ float s[NT];
@@ -723,11 +759,14 @@ __global__ void __launch_bounds__(NT) conv_gen_dw_reduce(const float *__restrict
   if (o < n) {
     const int z1 = min(Z, (w + 1) * per);
     int z = w * per;
+    float a = 0.f, b = 0.f, c = 0.f, d = 0.f;
     for (; z + 4 <= z1; z += 4) {
-      const float a = part[z * n + o], b = part[(z + 1) * n + o];
-      const float c = part[(z + 2) * n + o], d = part[(z + 3) * n + o];
-      v += a; v += b; v += c; v += d;
+      a += part[z * n + o];
+      b += part[(z + 1) * n + o];
+      c += part[(z + 2) * n + o];
+      d += part[(z + 3) * n + o];
     }
+    v = (a + b) + (c + d);
     for (; z < z1; z++) v += part[z * n + o];
   }
   s[threadIdx.x] = v;
@@ -883,6 +922,7 @@ int run_gen(ConvG g, const int q[13], bool dry) {
   if (dry) return 0;
   if (ttk_fail_direct_conv()) return -3;
   g.ck = p.ck;
+  g.close = !DX ? p.ck * g.HH * g.WW : g.C > 96 ? 10 : 4;
   g.cs = (int)p.cs;
   g.lda = (int)p.lda;
   g.ftiles = (int)p.ftiles;
