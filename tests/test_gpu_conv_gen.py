@@ -134,6 +134,29 @@ def test_conv_gen_nonfinite_stays_local(tlib, case):
         orc.conv2d_fwd(x, wbad, np.zeros(F, np.float32), sh, sw, ph, pw)))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("case", [CASES[k] for k in (1, 2, 3, 5, 6, 7, 8, 9)])
+def test_conv_gen_dx_nonfinite_weight(tlib, case, bad):
+    """The input gradient adds only the taps that reach an element: an infinite
+    or NaN weight changes the elements that it reaches, and none beside the
+    border that it does not (the padding is no product of its)."""
+    N, C, H, W, F, HH, WW, sh, sw, ph, pw = case
+    q, Ho, Wo = _q(case)
+    L = _lib()
+    w = rng.uniform(0.5, 1, (F, C, HH, WW)).astype(np.float32)
+    w[F - 1, C - 1, 0, 0] = bad
+    g = rng.uniform(0.5, 1, (N, F, Ho, Wo)).astype(np.float32)
+    x = np.zeros((N, C, H, W), np.float32)
+    dX, gd, wd = DevBuf(x.size), DevBuf.from_np(g), DevBuf.from_np(w)
+    check(L.ttk_conv_gen_dx(gd.ptr, wd.ptr, dX.ptr, q), "dx")
+    ref, got = orc.conv2d_bwd(x, w, g, sh, sw, ph, pw)[0], dX.to_np(x.shape)
+    fin = np.isfinite(ref)
+    assert not fin.all() and fin.any()
+    assert np.array_equal(np.isfinite(got), fin)
+    assert err(got[fin], ref[fin], F * HH * WW, 1.0, 1.0) <= TOL
+
+
 def test_conv_route():
     """Which kernel a convolution takes (no GPU needed)."""
     L = _lib()

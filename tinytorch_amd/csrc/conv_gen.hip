@@ -43,6 +43,7 @@
 // each with the taps that reach it: no product is formed with an inserted
 // zero.
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 #include "tt_rt.h"
 
@@ -323,6 +324,49 @@ __device__ __forceinline__ void add(f32x16 (&a)[MI][NJ], const f32x16 (&b)[MI][N
       for (int q = 0; q < 16; q++) a[i][j][q] += b[i][j][q];
 }
 
+// A wave's outputs of a 32 x P tile of the input gradient (WP pixels from wn * WP
+// on; of KW waves with the same pixels, the rows that wave wk stores), a lane an
+// element, from memory and the taps in range alone.  The arguments are read and
+// the tile found again here: kept for it through conv_gen_kernel's loop, they
+// took that loop's scalar registers (21 -> 48 spilled, 6-10 % slower).
+template <int P, int WP, int KW>
+__device__ __forceinline__ void dx_block_by_taps(int wn, int wk) {
+  typedef const __attribute__((address_space(4))) ConvG Args;
+  unsigned long long at = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
+  int bx = blockIdx.x, bz = blockIdx.z;
+  asm volatile("" : "+s"(at), "+s"(bx), "+s"(bz));
+  Args &g = *reinterpret_cast<Args *>(at);
+  const int a = bz / g.sw, H = g.H, W = g.W, C = g.C, F = g.F, taps = g.HH * g.WW;
+  const Axis ah = axis_dx(g.HH, g.sh, g.ph, g.OH, a);
+  const Axis aw = axis_dx(g.WW, g.sw, g.pw, g.OW, bz - a * g.sw);
+  const int pid = xcd_order(bx, gridDim.x), pt = pid / g.ftiles;
+  const int f0 = (pid - pt * g.ftiles) * 32, p0 = pt * P + wn * WP;
+  const int img = ah.no * aw.no, px = g.N * img;
+#pragma unroll 1
+  for (int e = threadIdx.x & 63; e < 32 * WP; e += 64) {
+    const int r = e / WP, f = f0 + r, p = p0 + e % WP;
+    if (f >= F || p >= px || (KW > 1 && (4 * (r >> 3) + (r & 3)) * KW / 16 != wk)) continue;
+    const int n = p / img, ho = (p - n * img) / aw.no, wo = p - n * img - ho * aw.no;
+    float v = 0.f;
+#pragma unroll 1
+    for (int c = 0; c < C; c++) {
+      const float *const gi = g.x + ((long)n * C + c) * H * W;
+      const float *const wi = g.w + ((long)c * F + f) * taps;
+      float s = 0.f;
+#pragma unroll 1
+      for (int i = 0; i < ah.n; i++)
+#pragma unroll 1
+        for (int j = 0; j < aw.n; j++) {
+          const int hi = ho + ah.lo + i, wj = wo + aw.lo + j;
+          if ((unsigned)hi < (unsigned)H && (unsigned)wj < (unsigned)W)
+            s += wi[(ah.k0 + i * ah.ks) * g.WW + aw.k0 + j * aw.ks] * gi[hi * W + wj];
+        }
+      v += s;
+    }
+    g.out[((long)n * F + f) * g.OH * g.OW + (ah.o0 + ho * ah.os) * g.OW + aw.o0 + wo * aw.os] = v;
+  }
+}
+
 // Forward (DX false) and input gradient (DX true).  Waves: WM x WN of them
 // tile BF = 32 MI WM output channels by P = 32 NJ WN pixels, and KW of them
 // share a tile's summed indices.  VA: 16-byte loads of the weights.
@@ -484,7 +528,10 @@ conv_gen_kernel(const ConvG g) {
 
   const bool ragged = nchunk && g.C % g.ck;
   if (nchunk) {
-    zero_lds(smem + asz, g.ck * g.cs, tid);  // the padding, which no load writes
+    // the padding, which no load writes (dX: the missing channels' weights too,
+    // whose sums are looked at below)
+    const int z0 = DX && f0 + BF > g.F ? 0 : asz;
+    zero_lds(smem + z0, asz - z0 + g.ck * g.cs, tid);
     __syncthreads();
   }
   for (int ch = 0; ch < nchunk; ch++) {
@@ -517,6 +564,22 @@ conv_gen_kernel(const ConvG g) {
     }
   } else {
     if (!nchunk) __syncthreads();  // the bias
+  }
+
+  // dX adds only the taps that reach an output; the slab's zeros stand for the
+  // others, and times an infinite or NaN weight they are not zero.  Such a weight
+  // leaves no sum of its output channel finite: a wave with a sum that is not
+  // forms its outputs again tap by tap.
+  if constexpr (DX) {
+    float z = 0.f;
+#pragma unroll
+    for (int q = 0; q < 16; q++)
+#pragma unroll
+      for (int j = 0; j < NJ; j++) z = __builtin_fmaf(acc[0][j][q], 0.f, z);
+    if (__ballot(z != 0.f)) {  // NaN
+      dx_block_by_taps<P, 32 * NJ, KW>(wn, wk);
+      return;
+    }
   }
 
   // ---- bias, relu, store: row 8 (q / 4) + 4 h + q % 4 of a block ----
