@@ -45,18 +45,49 @@ def test_ring_tiles(tlib, M, N, K, ta, tb):
         L.ttk_gemm_large(prev)
 
 
-@pytest.mark.parametrize("M,N,K,ta,tb", [
-    (2049, 1024, 300, 1, 0),    # 2048 rows and one of their own
-    (1000, 2049, 512, 0, 1),    # the same in columns
-    (1153, 2304, 301, 0, 0),    # 128x128 tiles, a ragged last row of them
-    (3329, 2300, 64, 0, 0),     # a second GEMM of a few tile rows
-    (300, 700, 2600, 0, 1),     # split K
-    (1024, 1024, 256, 1, 1),    # whole tiles, both transposed
-])
-def test_large_plan(tlib, M, N, K, ta, tb):
-    """Each outcome of the plan, and the entry without allocation: the same bits."""
+MID, RING, DIRECT, SPLIT, ROWS, COLS = range(6)  # ttk_gemm_plan_taken's outcomes
+
+
+def _taken(L):
+    L.ttk_gemm_plan_taken.restype = ctypes.c_long
+    return np.array([L.ttk_gemm_plan_taken(i) for i in range(6)])
+
+
+def _planned(tlib, M, N, K, ta, tb):
+    """One GEMM and the entry without allocation, the same bits; the plan's
+    outcomes of the first."""
+    before = _taken(tlib)
     c, (dA, dB) = _run(tlib, M, N, K, ta, tb)
+    got = _taken(tlib) - before
     out = DevBuf(M * N)
     check(tlib.tt_k_gemm_noalloc(M, N, K, dA.ptr, M if ta else K, ta, dB.ptr, K if tb else N, tb,
                                  out.ptr, N), "noalloc")
     assert np.array_equal(out.to_np((M * N,)), c)
+    return got
+
+
+@pytest.mark.parametrize("M,N,K,ta,tb,outcome", [
+    (2049, 1024, 300, 1, 0, MID),    # a last round of a few tiles, cheaper than a second GEMM
+    (1000, 2049, 512, 0, 1, MID),
+    (1153, 2304, 301, 0, 0, MID),
+    (3329, 2300, 64, 0, 0, RING),    # a ragged last row and column of 128x128 tiles
+    (300, 700, 2600, 0, 1, MID),     # few tiles: split K on 64x64 ones
+    (1024, 1024, 256, 1, 1, MID),    # whole tiles, both transposed
+    (1400, 1200, 4096, 0, 1, SPLIT),
+    (1400, 1200, 4095, 1, 0, SPLIT),  # 4-byte loads, a ragged last split
+    (4096, 4096, 64, 0, 0, DIRECT),
+])
+def test_large_plan(tlib, M, N, K, ta, tb, outcome):
+    """Each kernel that the plan gives a single GEMM to."""
+    got = _planned(tlib, M, N, K, ta, tb)
+    assert got[outcome] == 1 and got.sum() == 1, got
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K,cut", [(2049, 1024, 1000, ROWS), (1024, 2049, 1000, COLS),
+                                       (2051, 1024, 999, ROWS), (1024, 2051, 999, COLS)])
+def test_two_gemms(tlib, M, N, K, cut, ta, tb):
+    """The rows or columns past the last full round of tiles as a GEMM of their
+    own, from every layout of both operands, 16- and 4-byte loads."""
+    got = _planned(tlib, M, N, K, ta, tb)
+    assert got[cut] == 1 and got[ROWS] + got[COLS] == 1, got

@@ -16,7 +16,8 @@ rng = np.random.default_rng(31)
                                    (513, 2051, 300),    # rows of C off 16 bytes
                                    (2048, 2048, 130),   # 128x128 tiles
                                    (300, 1100, 900),    # split K: the reduction's epilogue
-                                   (2049, 1024, 150)])  # two GEMMs: a pass of its own
+                                   (2049, 1024, 150),   # a last round of a few tiles
+                                   (2049, 1024, 1000)])  # two GEMMs: a pass of its own
 def test_gemm_bias_relu(tlib, M, N, K):
     """Bit for bit the product (tt_k_gemm), then bias, then relu."""
     A = rng.uniform(-1, 1, (M, K)).astype(np.float32)

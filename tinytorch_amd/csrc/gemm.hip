@@ -1428,6 +1428,7 @@ int g_force_tile = -1, g_force_splits = -1;
 int g_direct = 1;  // direct-to-LDS 256x256 kernel enabled (tth_gemm_direct)
 int g_mid = 1;     // 64x64 direct-load kernel for plain GEMMs (tth_gemm_mid; 2: shared k tiles)
 int g_large = 1;   // the plan of large plain GEMMs (ttk_gemm_large)
+long g_plan_taken[6];  // its outcomes so far (ttk_gemm_plan_taken)
 int g_mid_force = 0;  // every plain GEMM of small size takes it too (tth_gemm_mid_force)
 int g_small = 1;   // 32x32 register kernel for small plain GEMMs (tth_gemm_small)
 int g_t16 = 1;     // 16x16 forward kernel for GEMMs below a full 32x32 grid (tth_gemm_t16)
@@ -2358,6 +2359,7 @@ int run(int M, int N, int K, Opnd A, Opnd B, float *C, long ldc, const float *bi
           g_red_hook = hook;
         }
       } nest(lp.m1 || lp.n1);
+      if (lp.m1 || lp.n1) g_plan_taken[lp.m1 ? 4 : 5]++;
       if (lp.m1) {
         Opnd A2 = A;
         A2.p += A_KC ? lp.m1 * A.ld : lp.m1;
@@ -2380,6 +2382,7 @@ int run(int M, int N, int K, Opnd A, Opnd B, float *C, long ldc, const float *bi
       }
       const BlockPlan bp = g_large == 2 ? BlockPlan{PK_RING, 1, (K + 63) / 64 * 64, 0}
                                         : plan_block(M, N, K, !v, dok);
+      g_plan_taken[bp.kind == PK_RING && bp.splits > 1 ? 3 : bp.kind]++;
       if constexpr (A_KC && B_NC) {
         // a layer's bias and relu in the tiles' stores
         RedHook *const h = g_red_hook;
@@ -2538,6 +2541,13 @@ extern "C" int ttk_gemm_large(int on) {
   const int prev = g_large;
   if (on >= 0) g_large = on;
   return prev;
+}
+
+// Diagnostics: how many GEMMs the plan has given to the 64x64 tiles (0), the
+// 128x128 tiles unsplit (1) and split over K (3) and the 256x256 tiles (2), each
+// block of two counted, and how many it has cut by rows (4) and by columns (5).
+extern "C" long ttk_gemm_plan_taken(int outcome) {
+  return outcome >= 0 && outcome < 6 ? g_plan_taken[outcome] : -1;
 }
 
 extern "C" int tth_gemm_mid_force(int on) {

@@ -52,6 +52,7 @@ int    ttk_gemm_bias_relu(int M, int N, int K, const float *A, const float *B, c
                           float *C, float *R);
 int    ttk_gemm_tn_colsum(int rows, int Kx, int N, const float *X, const float *G, float *dW);
 int    ttk_gemm_large(int on);          /* tuning: the plan of large GEMMs */
+long   ttk_gemm_plan_taken(int outcome);  /* diagnostics: what it came to */
 /* elementwise.hip: the split-K reduction of a GEMM (ws: S partial M x N
  * products, summed as gemm.hip's reduce_one does with zl lanes an element)
  * plus bias into C, and the softmax-CE of C's rows in the same launch:
