@@ -74,6 +74,31 @@ def test_softmax_small_rows(tlib):
         np.testing.assert_allclose(got[keep], e / e.sum(1, keepdims=True), rtol=1e-5)
 
 
+@pytest.mark.parametrize("rows,cols", [(300, 10), (300, 17), (300, 100), (300, 200), (300, 300),
+                                       (3073, 1)])
+def test_label_outside_the_columns(tlib, rows, cols):
+    """A label past the columns has no probability, whatever the row (of -inf:
+    1 / cols in each column), and its loss is log(1e-12) with the same bits
+    from every entry; a few of them alone make up the mean here."""
+    x = np.zeros((rows, cols), np.float32)
+    x[:2] = -np.inf
+    x[2:, 0] = 200.0  # loss 0 beside those rows
+    y = np.zeros(rows, np.int32)
+    y[:3] = (cols, cols + 1, -1)
+    dx, dl = DevBuf.from_np(x), DevBuf.from_np(y)
+    pr, se, me, lo = DevBuf(x.size), DevBuf(x.size), DevBuf(1), DevBuf(rows)
+    sc = ctypes.c_float(1.0)
+    check(tlib.tt_k_softmax_ce(dx.ptr, dl.ptr, pr.ptr, lo.ptr, se.ptr, rows, cols, sc), "ce")
+    got = lo.to_np()
+    np.testing.assert_allclose(got[:3], -np.log(1e-12), rtol=1e-6)
+    assert np.all(got[3:] == 0.0)
+    np.testing.assert_array_equal(pr.to_np((rows, cols))[:2], np.float32(1.0) / np.float32(cols))
+    np.testing.assert_array_equal(se.to_np((rows, cols))[:3], pr.to_np((rows, cols))[:3])
+    check(tlib.tt_k_softmax_ce_mean(dx.ptr, dl.ptr, pr.ptr, me.ptr, se.ptr, rows, cols, sc), "mean")
+    check(tlib.tt_k_ce_mean_rows(lo.ptr, lo.ptr, rows), "mean of the rows")
+    assert me.to_np()[0] == lo.to_np()[0]
+
+
 @pytest.mark.parametrize("rows,cols", [(40, 10), (513, 10), (700, 70)])
 @pytest.mark.parametrize("what", ["logits", "gradient", "stepped"])
 def test_second_backward_has_the_forward_seed(tlib, rows, cols, what):

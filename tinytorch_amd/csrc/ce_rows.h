@@ -92,6 +92,15 @@ __device__ __forceinline__ void ce_rows_block(const float *__restrict__ x, const
   ce_mean_tree(acc, part, loss_mean, rows);
 }
 
+// -log max(p, 1e-12), opaque to the optimiser: with a label out of range the
+// argument is the constant 1e-12, and a logf folded at compile time (correctly
+// rounded) can differ in the last bit from the device logf that ce_row runs
+__device__ __forceinline__ float ce_loss(float p) {
+  float a = fmaxf(p, 1e-12f);
+  asm volatile("" : "+v"(a));
+  return -logf(a);
+}
+
 // softmax_row_group: the probabilities of a row by a group of lanes; ce_row_group:
 // ce_row by a group of W lanes (W a power of two, the group's lanes
 // consecutive and all active), CPL columns a lane (cols <= W * CPL): lane q =
@@ -143,16 +152,11 @@ __device__ __forceinline__ float ce_row_group(const float (&x)[CPL], int y, int 
   for (int u = 0; u < CPL; u++) {
     const int j = q * CPL + u;
     sj[u] = (pj[u] - (j == y ? 1.0f : 0.0f)) * scale;
-    if (j == y) py = pj[u];
+    if (j == y && j < cols) py = pj[u];  // (a row of -inf has 1 / cols past its columns too)
   }
   // the lane that holds column y has its probability, the others 0 (and all
   // 0 for a label out of range): the largest over the group is p_y
 #pragma unroll
   for (int o = W / 2; o > 0; o >>= 1) py = fmaxf(py, __shfl_xor(py, o, W));
-  // opaque to the optimiser: with a label out of range the argument is the
-  // constant 1e-12, and a logf folded at compile time (correctly rounded)
-  // can differ in the last bit from the device logf that ce_row runs
-  float a = fmaxf(py, 1e-12f);
-  asm volatile("" : "+v"(a));
-  return -logf(a);
+  return ce_loss(py);
 }

@@ -268,7 +268,7 @@ ce_mean_probs_kernel(const float *__restrict__ probs, const LAB lab, float *__re
   float acc = 0.0f;
   for (int r = threadIdx.x; r < rows; r += 256) {
     const int y = lab[r];
-    acc += -logf(fmaxf(y >= 0 && y < cols ? probs[(long)r * cols + y] : 0.0f, 1e-12f));
+    acc += ce_loss(y >= 0 && y < cols ? probs[(long)r * cols + y] : 0.0f);
   }
   ce_mean_tree(acc, part, loss_mean, rows);
 }
