@@ -23,9 +23,10 @@ def _ref(x, y):
 
 @pytest.mark.parametrize("rows,cols", [(1, 1), (257, 10), (256, 17), (600, 32), (513, 33), (3072, 64),
                                        (3073, 65), (5, 128), (40, 129), (300, 255), (33, 256),
-                                       (65, 257), (9, 1000), (20000, 10)])
+                                       (65, 257), (9, 1000), (20000, 10), (3073, 1), (600, 2),
+                                       (4097, 4), (300, 5), (3075, 8), (257, 9)])
 def test_softmax_ce_rows(tlib, rows, cols):
-    """Every group width (16, 32, 64 lanes, a wavefront) and label form (two
+    """Every group width (1, 2, 16, 32, 64 lanes, a wavefront) and label form (two
     byte arrays in the arguments, device memory); fp32 exponentials and sums
     of `cols` terms stay within 1e-5 of float64."""
     from tinytorch_amd.torch_py import Node
@@ -62,7 +63,8 @@ def test_softmax_ce_rows(tlib, rows, cols):
 def test_softmax_small_rows(tlib):
     """Rows of up to 64 columns by groups of lanes, with a row of -inf."""
     rng = np.random.default_rng(3)
-    for rows, cols in ((1, 10), (17, 16), (5, 17), (100, 64), (3, 1)):
+    for rows, cols in ((1, 10), (17, 16), (5, 17), (100, 64), (3, 1), (513, 2), (257, 4), (9, 5),
+                       (260, 8), (18, 9)):
         x = rng.standard_normal((rows, cols)).astype(np.float32)
         x[rows // 2] = -np.inf
         d, y = DevBuf.from_np(x), DevBuf(x.size)
@@ -97,6 +99,44 @@ def test_label_outside_the_columns(tlib, rows, cols):
     check(tlib.tt_k_softmax_ce_mean(dx.ptr, dl.ptr, pr.ptr, me.ptr, se.ptr, rows, cols, sc), "mean")
     check(tlib.tt_k_ce_mean_rows(lo.ptr, lo.ptr, rows), "mean of the rows")
     assert me.to_np()[0] == lo.to_np()[0]
+
+
+def test_rows_past_one_launch(tlib):
+    """2^28 rows and more by 16 lanes a row are 2^32 work items, which one
+    launch does not take: 19 GB of logits and probabilities, all rows alike but
+    one on each side of every piece's edge (2^26 rows) and the last."""
+    rows, cols = 2 ** 28 + 3, 9
+    odd = sorted({k * 2 ** 26 + d for k in range(1, 5) for d in (-1, 0)} | {0, rows - 1})
+    x, y = DevBuf(rows * cols), DevBuf(rows * cols)
+    x.fill(1.0)
+    y.fill(7.0)
+    row = np.arange(cols, dtype=np.float32)
+    for r in odd:
+        check(tlib.tth_h2d(x.ptr + 4 * r * cols, row.ctypes.data, row.nbytes), "h2d")
+    e = np.exp(row.astype(np.float64))
+    p_odd, p_rest = e / e.sum(), np.full(cols, 1 / cols)
+
+    def rows_of(buf, r, n=cols):
+        out = np.empty(n, np.float32)
+        check(tlib.tth_d2h(out.ctypes.data, buf.ptr + 4 * r * n, out.nbytes), "d2h")
+        return out
+
+    def probabilities(buf):
+        for r in odd + [1, 2 ** 26 + 1, rows - 2]:
+            np.testing.assert_allclose(rows_of(buf, r), p_odd if r in odd else p_rest, rtol=1e-5)
+
+    check(tlib.tt_k_softmax_fwd(x.ptr, y.ptr, rows, cols), "softmax")
+    probabilities(y)
+    lab, lo, se = DevBuf(rows, np.int32), DevBuf(rows), DevBuf(rows * cols)
+    lab.fill(0.0)  # class 0
+    y.fill(7.0)
+    check(tlib.tt_k_softmax_ce(x.ptr, lab.ptr, y.ptr, lo.ptr, se.ptr, rows, cols,
+                               ctypes.c_float(0.5)), "ce")
+    probabilities(y)
+    for r in odd + [rows - 2]:
+        p = p_odd if r in odd else p_rest
+        np.testing.assert_allclose(rows_of(lo, r, 1), [-np.log(p[0])], rtol=1e-5)
+        np.testing.assert_allclose(rows_of(se, r), 0.5 * (p - np.eye(cols)[0]), rtol=1e-5, atol=4e-7)
 
 
 @pytest.mark.parametrize("rows,cols", [(40, 10), (513, 10), (700, 70)])

@@ -134,7 +134,7 @@ __device__ __forceinline__ void softmax_row_group(const float (&x)[CPL], int col
     float sum = 0.0f;
 #pragma unroll
     for (int c = 0; c < W * CPL; c++) {
-      const float t = __shfl(e[c % CPL], c / CPL, W);
+      const float t = W > 1 ? __shfl(e[c % CPL], c / CPL, W) : e[c % CPL];
       if (c < cols) sum += t;
     }
 #pragma unroll

@@ -135,9 +135,11 @@ struct SgdOp {
 // softmax, W lanes a row, CPL columns a lane (cols <= W * CPL): the bits of
 // one thread a row summing the columns in order (softmax_row_group), without
 // its serial loads -- one row of 10 took 4.3 us by one thread, 1.9 by 16 lanes.
+// Up to 8 columns 1 or 2 lanes a row, of 16 most would idle (a million rows of 2
+// 52.6 us by 16 lanes, 5.4 by one; of 8 53 and 18).
 template <int W, int CPL>
 __global__ void __launch_bounds__(256)
-softmax_group_kernel(const float *__restrict__ x, float *__restrict__ y, long rows, int cols) {
+softmax_group_kernel(const float *__restrict__ x, float *__restrict__ y, int rows, int cols) {
   const long r = (long)blockIdx.x * (256 / W) + threadIdx.x / W;
   const int q = threadIdx.x & (W - 1);
   if (r >= rows) return;
@@ -212,10 +214,10 @@ __global__ void __launch_bounds__(256)
 softmax_ce_group_kernel(const float *__restrict__ x, const LAB lab, float *__restrict__ probs,
                         float *__restrict__ loss, float *__restrict__ seed, int rows, int cols,
                         float scale) {
-  const int r = blockIdx.x * (256 / W) + threadIdx.x / W;
+  const long r = (long)blockIdx.x * (256 / W) + threadIdx.x / W;
   const int q = threadIdx.x & (W - 1);
   if (r >= rows) return;
-  const long o = (long)r * cols;
+  const long o = r * cols;
   float v[CPL], p[CPL], s[CPL];
 #pragma unroll
   for (int u = 0; u < CPL; u++) v[u] = q * CPL + u < cols ? x[o + q * CPL + u] : 0.0f;
@@ -903,18 +905,29 @@ int tt_k_sgd(float *w, const float *g, long n, float lr) {
   return run_map(n, a16(w) && a16(g), SgdOp{w, g, lr});
 }
 
+// f(first row, rows) for pieces of at most 2^22 workgroups of rpb rows: HIP
+// takes fewer than 2^32 work items a dimension.
+extern "C++" template <class F>
+static void for_rows(long rows, int rpb, F f) {
+  const long most = (1L << 22) * rpb;
+  for (long r = 0; r < rows; r += most) f(r, (int)(rows - r < most ? rows - r : most));
+}
+static unsigned groups(int rows, int rpb) { return (unsigned)((rows - 1) / rpb + 1); }
+
 int tt_k_softmax_fwd(const float *x, float *y, long rows, int cols) {
   if (rows <= 0 || cols <= 0) return 0;
-  if (cols <= 16 && rows <= 0x7fffffffL) {
-    hipLaunchKernelGGL((softmax_group_kernel<16, 1>), dim3((unsigned)((rows + 15) / 16)), dim3(256),
-                       0, stream(), x, y, rows, cols);
-  } else if (cols <= 64 && rows <= 0x7fffffffL) {
-    hipLaunchKernelGGL((softmax_group_kernel<16, 4>), dim3((unsigned)((rows + 15) / 16)), dim3(256),
-                       0, stream(), x, y, rows, cols);
-  } else {
-    hipLaunchKernelGGL(softmax_rowwave_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0,
-                       stream(), x, y, rows, cols);
-  }
+#define TT_SM(KERN, W_)                                                                      \
+  for_rows(rows, 256 / W_, [&](long r, int n) {                                              \
+    hipLaunchKernelGGL(KERN, dim3(groups(n, 256 / W_)), dim3(256), 0, stream(), x + r * cols, \
+                       y + r * cols, n, cols);                                               \
+  })
+  if (cols <= 2) TT_SM((softmax_group_kernel<1, 2>), 1);
+  else if (cols <= 4) TT_SM((softmax_group_kernel<1, 4>), 1);
+  else if (cols <= 8) TT_SM((softmax_group_kernel<2, 4>), 2);
+  else if (cols <= 16) TT_SM((softmax_group_kernel<16, 1>), 16);
+  else if (cols <= 64) TT_SM((softmax_group_kernel<16, 4>), 16);
+  else TT_SM(softmax_rowwave_kernel, 64);
+#undef TT_SM
   return launched();
 }
 
@@ -930,29 +943,37 @@ int tt_k_softmax_bwd(const float *s, const float *g, float *dx, long rows, int c
   return launched();
 }
 
+extern "C++" {
+static const int32_t *labels_from(const int32_t *lab, long r) { return lab + r; }
+template <class LAB>
+static const LAB &labels_from(const LAB &lab, long) { return lab; }  // (one piece)
+}
+
 extern "C++" template <class LAB>
 static void launch_ce_rows(const float *x, const LAB &lab, float *probs, float *loss, float *seed,
-                           int rows, int cols, float scale) {
-#define TT_CE(W_, CPL_)                                                                       \
-  hipLaunchKernelGGL((softmax_ce_group_kernel<W_, CPL_, LAB>),                                \
-                     dim3((unsigned)((rows + 256 / W_ - 1) / (256 / W_))), dim3(256), 0,      \
-                     stream(), x, lab, probs, loss, seed, rows, cols, scale)
-  if (cols <= 16) TT_CE(16, 1);
-  else if (cols <= 32) TT_CE(16, 2);
-  else if (cols <= 64) TT_CE(16, 4);
-  else if (cols <= 128) TT_CE(32, 4);
-  else if (cols <= 256) TT_CE(64, 4);
-  else
-    hipLaunchKernelGGL((softmax_ce_wave_kernel<LAB>), dim3((unsigned)((rows + 3) / 4)), dim3(256),
-                       0, stream(), x, lab, probs, loss, seed, rows, cols, scale);
+                           long rows, int cols, float scale) {
+#define TT_CE(KERN, W_)                                                                         \
+  for_rows(rows, 256 / W_, [&](long r, int n) {                                                 \
+    hipLaunchKernelGGL(KERN, dim3(groups(n, 256 / W_)), dim3(256), 0, stream(), x + r * cols,   \
+                       labels_from(lab, r), probs + r * cols, loss ? loss + r : loss,           \
+                       seed + r * cols, n, cols, scale);                                        \
+  })
+  if (cols <= 2) TT_CE((softmax_ce_group_kernel<1, 2, LAB>), 1);
+  else if (cols <= 4) TT_CE((softmax_ce_group_kernel<1, 4, LAB>), 1);
+  else if (cols <= 8) TT_CE((softmax_ce_group_kernel<2, 4, LAB>), 2);
+  else if (cols <= 16) TT_CE((softmax_ce_group_kernel<16, 1, LAB>), 16);
+  else if (cols <= 32) TT_CE((softmax_ce_group_kernel<16, 2, LAB>), 16);
+  else if (cols <= 64) TT_CE((softmax_ce_group_kernel<16, 4, LAB>), 16);
+  else if (cols <= 128) TT_CE((softmax_ce_group_kernel<32, 4, LAB>), 32);
+  else if (cols <= 256) TT_CE((softmax_ce_group_kernel<64, 4, LAB>), 64);
+  else TT_CE(softmax_ce_wave_kernel<LAB>, 64);
 #undef TT_CE
 }
 
 int tt_k_softmax_ce(const float *logits, const int32_t *labels, float *probs, float *loss_rows,
                     float *seed, long rows, int cols, float scale) {
   if (rows <= 0 || cols <= 0) return 0;
-  if (rows > 0x7fffffffL) return -1;
-  launch_ce_rows(logits, labels, probs, loss_rows, seed, (int)rows, cols, scale);
+  launch_ce_rows(logits, labels, probs, loss_rows, seed, rows, cols, scale);
   return launched();
 }
 
@@ -963,19 +984,19 @@ int ttk_ce_rows(const float *logits, const int32_t *host_labels, float *probs, f
   if (cols <= 255 && rows <= TT_CE_ARG_ROWS) {
     LabU8 la;
     lab_u8_fill(la, host_labels, rows, cols);
-    launch_ce_rows(logits, la, probs, rowloss, seed, (int)rows, cols, scale);
+    launch_ce_rows(logits, la, probs, rowloss, seed, rows, cols, scale);
     return launched();
   }
   if (cols <= 255 && rows <= BIG) {
     LabBytes<BIG> la;
     lab_u8_fill(la, host_labels, rows, cols);
-    launch_ce_rows(logits, la, probs, rowloss, seed, (int)rows, cols, scale);
+    launch_ce_rows(logits, la, probs, rowloss, seed, rows, cols, scale);
     return launched();
   }
   int32_t *dl = (int32_t *)ttrt_alloc(sizeof(int32_t) * (size_t)rows);
   int rc = dl && ttrt_h2d_async(dl, host_labels, sizeof(int32_t) * (size_t)rows) == 0 ? 0 : -2;
   if (rc == 0) {
-    launch_ce_rows(logits, (const int32_t *)dl, probs, rowloss, seed, (int)rows, cols, scale);
+    launch_ce_rows(logits, (const int32_t *)dl, probs, rowloss, seed, rows, cols, scale);
     rc = launched();
   }
   ttrt_free(dl);  // stream-ordered
