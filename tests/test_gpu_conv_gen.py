@@ -177,3 +177,55 @@ def test_conv_route():
         assert [route(big, k) for k in range(3)] == [0] * 3
     finally:
         L.tth_conv_lds(prev)
+
+
+@pytest.mark.parametrize("case,routes,direct", [
+    # the direct kernels of the forward and the weight gradient, the input
+    # gradient's (0: GEMM + col2im); whether a forward, a forward and weight
+    # gradient run direct
+    ((50, 24, 45, 37, 40, 5, 5, 2, 2, 2, 2), (2, 2, 2), (1, 1)),
+    ((37, 9, 55, 55, 13, 1, 1, 1, 1, 0, 0), (1, 1, 1), (1, 1)),    # 1x1: slab 10.6 us, chunks 11.7
+    ((14, 14, 18, 62, 6, 1, 1, 1, 1, 0, 0), (1, 1, 1), (1, 1)),    # 5.7 / 7.6
+    ((5, 119, 9, 15, 36, 5, 5, 2, 2, 1, 2), (2, 2, 0), (0, 0)),    # few tiles, 15 chunks: GEMM 17.7, chunks 43.5
+    ((1, 59, 23, 33, 9, 5, 5, 2, 2, 2, 2), (2, 2, 2), (0, 0)),     # 11.6 / 29.2
+    ((3, 109, 25, 47, 4, 5, 5, 2, 2, 2, 2), (2, 2, 2), (0, 0)),    # 22.1 / 45.2
+    ((12, 89, 11, 43, 39, 1, 1, 2, 2, 0, 0), (2, 1, 0), (0, 0)),   # 11.1 / 15.1
+])
+def test_conv_direct(case, routes, direct):
+    """Where the chunks would be the slower choice the GEMM or slab kernels
+    stay (no GPU needed)."""
+    L = _lib()
+    L.ttk_conv_direct.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    q = _q(case)[0]
+    assert tuple(L.ttk_conv_route(q, k) for k in range(3)) == routes
+    assert tuple(L.ttk_conv_direct(q, k) for k in range(2)) == direct
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [(5, 119, 9, 15, 36, 5, 5, 2, 2, 1, 2),   # GEMM throughout
+                                  (1, 59, 23, 33, 9, 5, 5, 2, 2, 2, 2),    # GEMM, dX by chunks
+                                  (12, 89, 11, 43, 39, 1, 1, 2, 2, 0, 0),
+                                  (14, 14, 18, 62, 6, 1, 1, 1, 1, 0, 0)])  # slab
+@pytest.mark.parametrize("train", [0, 1])
+def test_conv_mixed_routes(tlib, case, train):
+    """A layer whose products take different paths, with and without its weight
+    gradient (a forward that keeps its im2col matrix or not)."""
+    from tinytorch_amd.torch_py import Node
+    N, C, H, W, F, HH, WW, sh, sw, ph, pw = case
+    _, Ho, Wo = _q(case)
+    x = rng.uniform(-1, 1, (N, C, H, W)).astype(np.float32)
+    w = rng.uniform(-1, 1, (F, C, HH, WW)).astype(np.float32)
+    b = rng.uniform(-1, 1, F).astype(np.float32)
+    g = rng.uniform(-1, 1, (N, F, Ho, Wo)).astype(np.float32)
+    X, Wn, Bn = Node.leaf(x), Node.leaf(w, bool(train)), Node.leaf(b, bool(train))
+    y = X.conv2d(Wn, Bn, (sh, sw), (ph, pw))
+    y.backward(g)
+    rdx, rdw, rdb = orc.conv2d_bwd(x, w, g, sh, sw, ph, pw)
+    K = C * HH * WW
+    assert err(y.value(), orc.conv2d_fwd(x, w, b, sh, sw, ph, pw), K, 1.0, 1.0) <= TOL
+    assert err(X.grad(), rdx, F * HH * WW, 1.0, 1.0) <= TOL
+    if train:
+        assert err(Wn.grad(), rdw, N * Ho * Wo, 1.0, 1.0) <= TOL
+        assert err(Bn.grad(), rdb, N * Ho * Wo, 1.0, 1.0) <= TOL
+    for node in (y, X, Wn, Bn):
+        node.release()

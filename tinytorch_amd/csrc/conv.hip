@@ -42,6 +42,7 @@
 // 10x faster than per-lane scattered 4-byte ones.
 #include <hip/hip_runtime.h>
 #include <type_traits>
+#include <math.h>
 #include <stdint.h>
 #include <stdlib.h>
 #include "tt_rt.h"
@@ -3155,76 +3156,145 @@ extern "C" int tt_k_conv2d_chain_bwd(const float *dc2, const float *w2,
 
 extern "C" int ttk_fail_direct_conv(void) { return fail_direct(); }
 
+// ---- which kernel a convolution takes ----
+// The kernels here (the rows of every channel in LDS: "slab"), those of
+// conv_gen.hip (channel chunks), or im2col / col2im and a GEMM, by estimated
+// microseconds.  The estimates are fitted to 960 shapes (ttk_conv_gen_us says
+// which), on whole calls for the GEMM path: the ratio to the measured time has a
+// standard deviation of 0.13 for the slab kernels (0.06 for the tiled weight
+// gradient) and 0.16-0.22 for the GEMM path.  Where the slab kernel covers a
+// shape (else the GEMM), another is taken only if its estimate is 10 % and 1.5 us
+// lower.  Of the 960, 22 forwards, 22 forwards with their weight gradient and 11
+// input gradients are then more than 5 % slower than always slab, else GEMM, and
+// the geometric means over all of them are 1.17, 1.13 and 1.15 times as fast
+// (the best choice each time: 1.22, 1.20, 1.20; rules on channels, rows and
+// strides alone: 115, 116 and 86 slower and 1.14, 1.11, 1.08).
 namespace {
 
-// Estimated microseconds of the input gradient: the chunked kernel multiplies
-// 32 input channels whatever C is (95 TFLOP/s measured where its grid fills
-// the chip, and a chunk's round trip of 1 us and 10 ns an index where it does
-// not); the GEMM of the column gradient wastes nothing (60 TFLOP/s) but moves
-// the C * taps * pixels matrix out and back through col2im (measured: 64 x 8 x
-// 30 x 30 -> 200: 95 against 53 us; 24 x 16 x 16 x 16 -> 100, 5 x 5: 39 against
-// 27; 404 x 16 x 16 x 16 -> 32, 5 x 5: 67 against 111; 32 x 64 x 56 x 56 -> 128:
-// 168 against 253).
-double dx_chunk_us(const Geo &g, int N) {
-  const double taps = (double)g.HH * g.WW, px = (double)N * g.Ho * g.Wo;
-  const double work = 2.0 * ((g.C + 31) / 32 * 32) * g.F * taps * px / 95e6;
-  const double serial = (g.F + 7) / 8 * (1 + 0.08 * taps / (g.sh * g.sw));
-  return (work > serial ? work : serial) + 6;
-}
-double dx_gemm_us(const Geo &g, int N) {
-  const double taps = (double)g.HH * g.WW, px = (double)N * g.Ho * g.Wo;
-  return 2.0 * g.C * g.F * taps * px / 60e6 + 8.0 * g.C * taps * px / 2.5e6 + 12;
-}
-// (the slab kernel, TFLOP/s of padded channels: 60 with 3x3 taps, 64 x 4 x 30 x
-// 30 -> 64 41 us against the GEMM's 23; else 45, 404 x 16 x 16 x 16 -> 32, 5 x
-// 5: 119 us)
-double dx_slab_us(const Geo &g, int N) {
-  const double taps = (double)g.HH * g.WW, px = (double)N * g.Ho * g.Wo;
-  const double work = 2.0 * ((g.C + 31) / 32 * 32) * g.F * taps * px;
-  return is_k3(g) ? work / 60e6 + 4 : work / 45e6 + 8;
+double slab_us(const Geo &g, int N, bool flip) {
+  const FwdPlan p = plan_fwd(g, N, flip);
+  const double per = tt_per_cu((double)N * p.chunks * ((g.F + 31) / 32));
+  const double quads = (g.K + 7) / 8 * (double)p.pb / p.ks;
+  const double resident = p.lds > LDS_MAX / 2 ? 1 : p.lds > LDS_MAX / 3 || !flip ? 2 : 2.6;
+  const double rounds = per > resident ? per / resident : 1;
+  return (flip ? 0.4 + 3.3 * rounds : 1.1 + 2.44 * rounds) +
+         per * (quads * (flip ? is_k3(g) ? 0.15 : 0.227 : is_k3(g) ? 0.157 : 0.194) + p.lds * 8.5e-5);
 }
 
-}  // namespace
-
-// Which kernel a convolution of this geometry takes (what: 0 forward, 1
-// weight gradient, 2 input gradient): TT_ROUTE_SLAB the kernels here that
-// hold the rows of every channel in LDS, TT_ROUTE_CHUNK those of
-// conv_gen.hip, 0 neither (im2col + GEMM).  Where both cover a shape, the
-// slab kernels are the faster ones for 3x3 stride-1 taps with 16-byte rows
-// (128 x 32 x 16 x 16 -> 64: forward 17.7 us against 21.0, dX 16.9 / 27; with
-// 14-float rows 17.0 / 14.5 and 15.1 / 23), for few channels (128 x 3 x 32
-// x 32 -> 32: 10.2 / 17; dW of 64 x 6 x 30 x 30 -> 64: 24.7 / 38), and the
-// tiled weight gradient where its units fit (25.1 / 37; 404 x 16 x 16 x 16 ->
-// 32, 5 x 5: 60 / 68) except over many filters and taps (32 x 64 x 56 x 56 ->
-// 128: 212 / 190); elsewhere the chunked ones (50 x 24 x 45 x 37 -> 40, 5 x 5,
-// stride 2: forward 72 / 31; 404 x 16 x 16 x 16 -> 32, 5 x 5: dX 119 / 67; 41 x
-// 41 x 64 x 63 -> 26, stride 2: dW 82 / 38).
-namespace {
-
-int conv_route(const int q[13], int what) {
-  const int N = q[0], C = q[1], H = q[2], W = q[3], F = q[4], HH = q[5], WW = q[6], sh = q[7],
-            sw = q[8], ph = q[9], pw = q[10], Ho = q[11], Wo = q[12];
-  if (!g_lds_conv || !geo_ok(N, C, H, W, F, HH, WW, sh, sw, ph, pw, Ho, Wo)) return 0;
-  const Geo g{C, H, W, HH, WW, sh, sw, ph, pw, Ho, Wo, F, C * HH * WW};
-  const bool slab = tt_k_conv2d_lds_plan(N, C, H, W, F, HH, WW, sh, sw, ph, pw, Ho, Wo) >> what & 1;
-  bool keep;   // the slab kernel where it covers the shape
-  bool chunk;  // the chunked one covers it
-  if (what == 0) {
-    keep = C < 8 || (is_k3(g) && sh == 1 && sw == 1 &&
-                     (W % 4 == 0 || (slab && pool_fusable(g, plan_fwd(g, N, false)))));
-    chunk = ttk_conv_gen_fwd(nullptr, nullptr, nullptr, nullptr, nullptr, q) == 0;
-  } else if (what == 1) {
-    keep = C < 8 || (g_dwt && plan_dwt(g, N).tg && (long)F * g.K < 65536);
-    chunk = ttk_conv_gen_dw(nullptr, nullptr, nullptr, nullptr, q) == 0;
-  } else {
-    chunk = ttk_conv_gen_dx(nullptr, nullptr, nullptr, q) == 0;
-    const double never = 1e30, tc = chunk ? dx_chunk_us(g, N) : never, tg = dx_gemm_us(g, N),
-                 ts = slab ? dx_slab_us(g, N) : never;
-    keep = slab && (is_k3(g) || ts <= tc);  // 3x3: faster than the chunked one, above
-    if (tg < (keep ? ts : tc)) return 0;
+double dw_slab_us(const Geo &g, int N) {
+  const double MB = 4e-6;
+  const DwtPlan t = plan_dwt(g, N);
+  if (g_dwt && t.tg) {
+    const double per = tt_per_cu((double)t.units * t.nts * t.nfb);
+    const double work = (double)t.ntgw * t.tg * t.rc * g.Wo / 2;
+    double resident = (double)(LDS_MAX / t.lds);
+    if (resident > 5.6) resident = 5.6;
+    return 5.1 + 1.72 * (per > resident ? per / resident : 1) + per * (work * 0.009 + t.lds * 3.1e-5) +
+           0.51 * MB * t.units * t.nfb * (t.jbp * 1024.0 + 32);
   }
-  if (slab && (keep || !chunk)) return TT_ROUTE_SLAB;
-  return chunk ? TT_ROUTE_CHUNK : 0;
+  const DwPlan p = plan_dw(g, N);
+  const double resident = p.lds > LDS_MAX / 2 ? 1 : 2;
+  if (p.var >= 10) {
+    const double grid = (double)N * p.chunks * ((g.F + 31) / 32), jb = (g.K + 31) / 32;
+    const double per = tt_per_cu(grid);
+    return 6.0 + 2.28 * (per > resident ? per / resident : 1) +
+           per * (jb * p.ch / 2 * 0.0214 + p.lds * 4.4e-5) + 0.27 * MB * grid * (jb * 1024 + 32);
+  }
+  const double jb = (g.K + 15) / 16;
+  const double per = tt_per_cu((double)N * p.chunks * ((g.F + 16 * p.fs - 1) / (16 * p.fs)));
+  return 3.1 + 3.44 * (per > resident ? per / resident : 1) +
+         per * (p.fs * jb * p.ch / 8 * 0.0223 + p.lds * 9.2e-5) +
+         0.37 * MB * N * p.chunks * (double)g.F * (g.K + 1);
+}
+
+// what: 0 forward (keep: its im2col matrix too), 1 weight gradient from a kept
+// one, 2 input gradient
+double gemm_us(const Geo &g, int N, int what, bool keep) {
+  auto up = [](double v) { return ceil(v / 64) * 64; };
+  const double px = (double)N * g.Ho * g.Wo, col = 4e-6 * g.K * px;  // MB
+  const double io = 4e-6 * ((double)N * g.C * g.H * g.W + g.F * px);
+  const double f = g.F <= 16 ? 16 : g.F <= 32 ? 32 : up(g.F);
+  const double m = what == 2 ? up(g.K) : f, n = what == 1 ? up(g.K) : up(px);
+  const double k = what == 0 ? g.K : what == 1 ? px : g.F;
+  const double tiles = m * n / 4096, gf = 2e-9 * m * n * k;
+  const double serial = k * (tiles > 256 ? 256 / tiles : 1);  // the summed index of few tiles
+  const bool odd = g.Ho * g.Wo % 4 || g.K % 4, k1 = g.HH * g.WW == 1, strided = g.sh * g.sw > 1;
+  const bool implicit = col > 268;  // no im2col matrix
+  if (what == 0)
+    return (keep ? 11.2 : 9.1) - (k1 ? 1.5 : 0) + (implicit ? 0 : col * (k1 ? 0.05 : 0.34)) +
+           11.4 * gf * (odd ? 1.29 : 1) + 0.46 * io + 0.0057 * serial;
+  if (what == 1)
+    return 7.2 - (k1 ? 1.3 : 0) + (implicit ? 0 : col * 0.17) +
+           11.3 * gf * (odd ? 1.2 : 1) * (implicit ? 1.5 : 1) + 1.0;
+  return 12.0 - (k1 ? 4.8 : 0) + (implicit ? 0 : col * 0.55 * (k1 ? 1.55 : strided ? 2.9 : 1)) +
+         10.2 * gf * (odd ? 1.12 : 1) * (implicit ? 1.8 : 1) + 0.018 * serial;
+}
+
+constexpr double NEVER = 1e30;
+bool surely(double us, double than) { return us + 1.5 < 0.9 * than; }
+
+struct ConvCost {
+  bool slab, chunk;  // covered
+  double us;         // of the one taken
+  int route;
+};
+
+// the direct kernel of the forward (0) or the weight gradient (1)
+ConvCost conv_cost(const Geo &g, const int q[13], int what) {
+  const int N = q[0];
+  ConvCost c;
+  c.slab = tt_k_conv2d_lds_plan(N, q[1], q[2], q[3], q[4], q[5], q[6], q[7], q[8], q[9], q[10],
+                                q[11], q[12]) >> what & 1;
+  c.chunk = (what == 0   ? ttk_conv_gen_fwd(nullptr, nullptr, nullptr, nullptr, nullptr, q)
+             : what == 1 ? ttk_conv_gen_dw(nullptr, nullptr, nullptr, nullptr, q)
+                         : ttk_conv_gen_dx(nullptr, nullptr, nullptr, q)) == 0;
+  const Geo gx{g.F, g.Ho, g.Wo, g.HH, g.WW, 1, 1, g.HH - 1 - g.ph, g.WW - 1 - g.pw, g.H, g.W, g.C,
+               g.F * g.HH * g.WW};
+  const double ts = !c.slab ? NEVER : what == 0 ? slab_us(g, N, false) : what == 1 ? dw_slab_us(g, N)
+                                                                                   : slab_us(gx, N, true);
+  const double tc = c.chunk ? ttk_conv_gen_us(q, what) : NEVER;
+  // what a fused pool or a deferred reduction joins stays there; of the tiled
+  // weight gradient all but many filters and taps (32 x 64 x 56 x 56 -> 128: 212
+  // / 205 us, and 1.0e-6 / 1.9e-7 from the 64-bit result)
+  const bool tiled = what == 1 && g_dwt && plan_dwt(g, N).tg;
+  const bool wide = tiled && (long)g.F * g.K >= 65536;
+  // Chunks are at least 8 channels: with fewer (of 316 forwards 18 were 10 %
+  // faster by chunks, 264 slower), 1x1 forwards of fewer than 32 (10 of 117, 87)
+  // and other 1x1 products (of 250 34, 151) stay too.
+  const bool one = g.HH * g.WW == 1;
+  const bool keep = what == 0   ? g.C < 8 || (one && g.C < 32) ||
+                                    (is_k3(g) && g.sh == 1 && g.sw == 1 &&
+                                     pool_fusable(g, plan_fwd(g, N, false)))
+                    : what == 1 ? g.C < 8 || one || tiled
+                                : one;
+  c.route = c.slab && !(wide && c.chunk) && (keep || !surely(tc, ts)) ? TT_ROUTE_SLAB
+            : c.chunk                                                ? TT_ROUTE_CHUNK
+                                                                     : 0;
+  c.us = c.route == TT_ROUTE_SLAB ? ts : tc;
+  return c;
+}
+
+// what: 0, 1 the direct kernel; 2 the input gradient's, 0 the GEMM; 3, 4
+// whether the forward, the forward and the weight gradient, run direct
+int conv_route(const int q[13], int what) {
+  const int N = q[0];
+  if (!g_lds_conv || !geo_ok(N, q[1], q[2], q[3], q[4], q[5], q[6], q[7], q[8], q[9], q[10], q[11],
+                             q[12]))
+    return 0;
+  const Geo g{q[1], q[2], q[3], q[5], q[6], q[7], q[8], q[9], q[10], q[11], q[12], q[4],
+              q[1] * q[5] * q[6]};
+  if (what < 2) return conv_cost(g, q, what).route;
+  if (what == 2) {
+    const ConvCost x = conv_cost(g, q, 2);
+    const double tg = gemm_us(g, N, 2, false);
+    return (x.slab ? surely(tg, x.us) : !surely(x.us, tg)) ? 0 : x.route;
+  }
+  const ConvCost f = conv_cost(g, q, 0);
+  if (what == 3) return f.route && (f.slab || surely(f.us, gemm_us(g, N, 0, false)));
+  const ConvCost w = conv_cost(g, q, 1);
+  return f.route && w.route &&
+         ((f.slab && w.slab) ||
+          surely(f.us + w.us, gemm_us(g, N, 0, true) + gemm_us(g, N, 1, true)));
 }
 
 struct ConvRoute {
@@ -3232,10 +3302,16 @@ struct ConvRoute {
 };
 TTPlanCache<ConvRoute> g_routes;
 
+int cached_route(const int q[13], int what) {
+  return g_routes
+      .get(q, what + 5 * (g_lds_conv + 2 * g_dwt), [&] { return ConvRoute{conv_route(q, what)}; })
+      .r;
+}
+
 }  // namespace
 
 extern "C" int ttk_conv_route(const int q[13], int what) {
-  return g_routes
-      .get(q, what + 3 * (g_lds_conv + 2 * g_dwt), [&] { return ConvRoute{conv_route(q, what)}; })
-      .r;
+  return what < 0 || what > 2 ? 0 : cached_route(q, what);
 }
+
+extern "C" int ttk_conv_direct(const int q[13], int train) { return cached_route(q, train ? 4 : 3); }

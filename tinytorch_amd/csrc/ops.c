@@ -496,9 +496,9 @@ Tensor *tt_conv2d_keepcol_ex(const Tensor *a, const Tensor *w, const Tensor *b, 
     }
     const int Kc = C * HH * WW;
     const long Ncol = (long)N * Ho * Wo;
-    /* direct convolution: taken when a direct kernel also covers the weight
+    /* direct convolution: taken when it is the faster together with the weight
      * gradient the caller will ask for (that reads x, so no col is kept) */
-    const int direct = ttk_conv_route(q, 0) && (!col_out || ttk_conv_route(q, 1));
+    const int direct = ttk_conv_direct(q, col_out != NULL);
     if (direct && defer && g_conv_relu) {
         tt_flush_pending();
         tt_pend.out = out;

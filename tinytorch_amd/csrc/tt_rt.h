@@ -149,7 +149,16 @@ int    ttk_conv_gen_dw(const float *gr, const float *x, float *dw, float *db, co
 /* tuning: force the plans (tile, channels a chunk, dW tile, splits; -1 / 0:
  * automatic) */
 void   ttk_conv_gen_force(int tile, int ck, int dw, int splits);
-/* conv.hip: the kernel of a convolution (what: 0 forward, 1 dW, 2 dX) */
+double ttk_conv_gen_us(const int q[13], int what);
+/* the workgroups of a grid that the busiest of 256 CUs takes */
+static inline double tt_per_cu(double grid) {
+  const double x = grid / 256;
+  return x > 4 ? x + 0.5 : x > 3 ? 4 : x > 2 ? 3 : x > 1 ? 2 : 1;
+}
+/* conv.hip: the kernel of a convolution (what: 0 forward, 1 dW: among the
+ * direct ones; 2 dX: 0 where the GEMM is faster), and whether the forward runs
+ * direct (train: its weight gradient too, without a kept im2col) */
+int    ttk_conv_direct(const int q[13], int train);
 #define TT_ROUTE_SLAB 1
 #define TT_ROUTE_CHUNK 2
 int    ttk_conv_route(const int q[13], int what);
