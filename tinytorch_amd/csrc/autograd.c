@@ -743,14 +743,20 @@ AGNode *ag_softmax_ce(AGNode *logits, const int *labels, long rows) {
         tt_release(probs); tt_release(seed); tt_release(loss); free(hlab);
         return NULL;
     }
-    /* the rows' softmax-CE in one launch; the mean loss a recipe of the row
-     * losses, as above */
-    Tensor *rl = tt_empty_dev(&rows, 1);
-    const int ok = probs && seed && loss && hlab && rl &&
-                   ttk_ce_rows(x, hlab, probs->dev, seed->dev, rl->dev, rows, cols,
-                               1.0f / (float)rows) == 0 &&
-                   (tt_lazy_ce_mean(loss, rl) == 0 ||
-                    tt_k_ce_mean_rows(rl->dev, loss->dev, (int)rows) == 0);
+    /* one workgroup's rows: the mean loss in the same launch (a read of it by
+     * itself costs another: 40 x 10 with its backward and the loss read 24.0 us,
+     * 27.7 with the recipe); else the rows' softmax-CE in one launch and the mean
+     * loss a recipe of the row losses, as above */
+    const int small = rows <= 256 && cols <= 32;
+    Tensor *rl = small ? NULL : tt_empty_dev(&rows, 1);
+    const float scale = 1.0f / (float)rows;
+    const int ok =
+        probs && seed && loss && hlab &&
+        (small ? tt_k_softmax_ce_mean_hostlab(x, hlab, probs->dev, loss->dev, seed->dev, rows,
+                                              cols, scale) == 0
+               : rl && ttk_ce_rows(x, hlab, probs->dev, seed->dev, rl->dev, rows, cols, scale) == 0 &&
+                     (tt_lazy_ce_mean(loss, rl) == 0 ||
+                      tt_k_ce_mean_rows(rl->dev, loss->dev, (int)rows) == 0));
     tt_release(rl);
     free(hlab);
     if (!ok) {

@@ -3164,11 +3164,12 @@ extern "C" int ttk_fail_direct_conv(void) { return fail_direct(); }
 // standard deviation of 0.13 for the slab kernels (0.06 for the tiled weight
 // gradient) and 0.16-0.22 for the GEMM path.  Where the slab kernel covers a
 // shape (else the GEMM), another is taken only if its estimate is 10 % and 1.5 us
-// lower.  Of the 960, 22 forwards, 22 forwards with their weight gradient and 11
-// input gradients are then more than 5 % slower than always slab, else GEMM, and
-// the geometric means over all of them are 1.17, 1.13 and 1.15 times as fast
-// (the best choice each time: 1.22, 1.20, 1.20; rules on channels, rows and
-// strides alone: 115, 116 and 86 slower and 1.14, 1.11, 1.08).
+// lower, and shapes of few products are not weighed at all (conv_cost).  Of the
+// 960, 10 forwards, 5 forwards with their weight gradient and 8 input gradients
+// are then more than 5 % slower than always slab, else GEMM, and the geometric
+// means over all of them are 1.17, 1.12 and 1.15 times as fast (the best choice
+// each time: 1.22, 1.20, 1.20; rules on channels, rows and strides alone: 115,
+// 116 and 86 slower and 1.14, 1.11, 1.08).
 namespace {
 
 double slab_us(const Geo &g, int N, bool flip) {

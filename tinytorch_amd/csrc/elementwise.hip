@@ -624,6 +624,25 @@ ce_mean_rows_kernel(const float *__restrict__ rowloss, float *__restrict__ loss,
   ce_mean_tree(acc, part, loss, rows);
 }
 
+// the sum of a workgroup's share of the rows
+__global__ void __launch_bounds__(256)
+ce_sum_rows_kernel(const float *__restrict__ rowloss, float *__restrict__ sums, int rows) {
+  __shared__ float part[256];
+  float acc = 0.0f;
+  for (long r = (long)blockIdx.x * 256 + threadIdx.x; r < rows; r += (long)gridDim.x * 256)
+    acc += rowloss[r];
+  ce_mean_tree(acc, part, sums + blockIdx.x, 1);
+}
+
+// loss = the sum of n partial sums / rows
+__global__ void __launch_bounds__(256)
+ce_mean_sums_kernel(const float *__restrict__ sums, float *__restrict__ loss, int n, int rows) {
+  __shared__ float part[256];
+  float acc = 0.0f;
+  for (int r = threadIdx.x; r < n; r += 256) acc += sums[r];
+  ce_mean_tree(acc, part, loss, rows);
+}
+
 // C = A * B + bias for a skinny B (N <= MAXN columns): one workgroup per
 // row of A.  Thread t forms the N dot-product pieces over k = t, t + 256, ...
 // (fused multiply-adds, in k order), the 256 pieces of each column are added
@@ -1232,6 +1251,18 @@ extern "C" int ttk_reduce_ce(const float *ws, float *C, int M, int N, int S, int
 
 extern "C" int tt_k_ce_mean_rows(const float *rowloss, float *loss, int rows) {
   if (rows <= 0) return -1;
+  // past TT_CE_MEAN_MAX_ROWS 16 rows a thread, then the workgroups' sums (a
+  // softmax-CE of 65536 x 10 and its backward with the loss read: by one
+  // workgroup 111 us, so 59; of a million rows 1309, 401)
+  const int nb = rows > TT_CE_MEAN_MAX_ROWS ? (rows - 1) / 4096 + 1 : 1;
+  float *sums = nb > 1 ? (float *)ttrt_alloc(sizeof(float) * (size_t)nb) : nullptr;
+  if (sums) {
+    hipLaunchKernelGGL(ce_sum_rows_kernel, dim3((unsigned)nb), dim3(256), 0, stream(), rowloss, sums,
+                       rows);
+    hipLaunchKernelGGL(ce_mean_sums_kernel, dim3(1), dim3(256), 0, stream(), sums, loss, nb, rows);
+    ttrt_free(sums);  // stream-ordered
+    return launched();
+  }
   hipLaunchKernelGGL(ce_mean_rows_kernel, dim3(1), dim3(256), 0, stream(), rowloss, loss, rows);
   return launched();
 }
