@@ -989,7 +989,7 @@ struct MidOperand {
   // R+15 of one chunk) touches every bank once (8-k rows: rows 8 apart would
   // share banks, so their two chunks swap)
   __device__ __forceinline__ static int swz(int R) {
-    return BK == 8 ? (R >> 3) & 1 : BK == 16 ? (R >> 1) & 3 : BK == 32 ? (R >> 1) & 7 : R & 15;
+    return BK == 8 ? (R >> 3) & 1 : BK == 32 ? (R >> 1) & 7 : R & 15;
   }
   unsigned voff[NL];
   const float *p;
@@ -2336,8 +2336,12 @@ int run(int M, int N, int K, Opnd A, Opnd B, float *C, long ldc, const float *bi
   Plan p = plan(M, N, K > 0 ? K : 1);
   if constexpr (!A_PERM && !B_PERM && !B_I2C && EPI == EPI_STORE) {
     // from 0.5 GFLOP: the kernel, split and, past the last full round of
-    // tiles, the second GEMM that plan_large picks
-    const bool large = 2.0 * M * N * K >= (double)(1L << 29) && N > 16 && M > 16;
+    // tiles, the second GEMM that plan_large picks.  Not up to K = 64, where the
+    // stores of C are most of the time and the tiles' rings of four stages never
+    // fill: of 62 such shapes 24 were slower than by the rules below (8000 x 7936 x
+    // 64 113 / 130 us, 11499 x 3969 x 31 65 / 105), 32 faster and the geometric
+    // mean 1.03; from 80 to 200 of 51 2 slower, 44 faster, 1.21.
+    const bool large = 2.0 * M * N * K >= (double)(1L << 29) && N > 16 && M > 16 && K > 64;
     if (((large && g_large && g_mid == 1 && !g_mid_force) || g_large == 2) && g_force_tile < 0 &&
         g_force_splits < 0 && K > 0 && A.ld <= (1L << 22) && B.ld <= (1L << 22) &&
         !(g_large == 1 && small_ok<A_KC, B_NC>(M, N, K, A, B))) {
