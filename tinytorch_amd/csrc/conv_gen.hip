@@ -367,21 +367,21 @@ __device__ __forceinline__ void dx_block_by_taps(int wn, int wk) {
   }
 }
 
-// Forward (DX false) and input gradient (DX true).  Waves: WM x WN of them
-// tile BF = 32 MI WM output channels by P = 32 NJ WN pixels, and KW of them
-// share a tile's summed indices.  VA: 16-byte loads of the weights.
+// Forward (DX false) and input gradient (DX true).  Waves: WN of them tile BF =
+// 32 output channels by P = 32 NJ WN pixels, and KW of them share a tile's
+// summed indices.  VA: 16-byte loads of the weights.
 //
 // Bound: the matrix pipe; staging of the next chunk runs under it.
-template <int WM, int WN, int MI, int NJ, int KW, bool DX, bool VA>
+template <int WN, int NJ, int KW, bool DX, bool VA>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2)))
 conv_gen_kernel(const ConvG g) {
-  static_assert(WM * WN * KW == NT / 64, "four waves");
-  constexpr int BF = 32 * MI * WM, P = 32 * NJ * WN;
+  static_assert(WN * KW == NT / 64, "four waves");
+  constexpr int BF = 32, P = 32 * NJ * WN;
   extern __shared__ __attribute__((aligned(16))) float smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, h = lane >> 5;
-  const int wk = wave / (WM * WN), wm = (wave / WN) % WM, wn = wave % WN;
+  const int wk = wave / WN, wn = wave % WN;
 
   Axis ah, aw;
   if constexpr (DX) {
@@ -504,23 +504,23 @@ conv_gen_kernel(const ConvG g) {
                      : -1;
   }
 
-  f32x16 acc[MI][NJ];
+  f32x16 acc[1][NJ];
   clear(acc);
 
   auto multiply = [&](int ch) {
     const float *const as = smem;
     const char *const xs = reinterpret_cast<const char *>(as + asz);
     const int kh = (min(g.ck, g.C - ch * g.ck) * T + 7) / 8 * 4;  // indices a lane half
-    const float *const al = as + (wm * MI * 32 + l32) * lda + h * kh;
+    const float *const al = as + l32 * lda + h * kh;
     const int *const tl = tab + h * kh;
     for (int q = 4 * wk; q < kh;) {
       const int end = min(kh, q + 4 * KW * g.close);
-      f32x16 part[MI][NJ];
+      f32x16 part[1][NJ];
       clear(part);
       for (; q < end; q += 4 * KW) {
-        float a[MI][4], bb[NJ][4];
-        read_quad<MI, NJ>(a, bb, al + q, 32 * lda, xs, pix, tl + q);
-        mul_quad<MI, NJ>(a, bb, part);
+        float a[1][4], bb[NJ][4];
+        read_quad<1, NJ>(a, bb, al + q, 0, xs, pix, tl + q);
+        mul_quad<1, NJ>(a, bb, part);
       }
       add(acc, part);
     }
@@ -548,7 +548,7 @@ conv_gen_kernel(const ConvG g) {
 
   // ---- the KW waves' sums of a tile, added in wave order ----
   if constexpr (KW > 1) {
-    static_assert(WM * MI == 1 && NJ == 1, "one 32 x 32 block a wave");
+    static_assert(NJ == 1, "one 32 x 32 block a wave");
     __syncthreads();
     float *const red = smem + wave * 1024;
 #pragma unroll
@@ -585,22 +585,20 @@ conv_gen_kernel(const ConvG g) {
   // ---- bias, relu, store: row 8 (q / 4) + 4 h + q % 4 of a block ----
   const int ohw = g.OH * g.OW;
 #pragma unroll
-  for (int i = 0; i < MI; i++)
+  for (int q = 0; q < 16; q++) {
+    if (KW > 1 && (q * KW) / 16 != wk) continue;
+    const int fl = 8 * (q >> 2) + 4 * h + (q & 3);
+    if (f0 + fl >= g.F) continue;
+    const float bv = bias[fl];
+    const long fo = (long)(f0 + fl) * ohw;
 #pragma unroll
-    for (int q = 0; q < 16; q++) {
-      if (KW > 1 && (q * KW) / 16 != wk) continue;
-      const int fl = (wm * MI + i) * 32 + 8 * (q >> 2) + 4 * h + (q & 3);
-      if (f0 + fl >= g.F) continue;
-      const float bv = bias[fl];
-      const long fo = (long)(f0 + fl) * ohw;
-#pragma unroll
-      for (int j = 0; j < NJ; j++) {
-        if (opix[j] < 0) continue;
-        const float v = acc[i][j][q] + bv;
-        g.out[fo + opix[j]] = v;
-        if (g.rout) g.rout[fo + opix[j]] = v > 0.f ? v : 0.f;
-      }
+    for (int j = 0; j < NJ; j++) {
+      if (opix[j] < 0) continue;
+      const float v = acc[0][j][q] + bv;
+      g.out[fo + opix[j]] = v;
+      if (g.rout) g.rout[fo + opix[j]] = v > 0.f ? v : 0.f;
     }
+  }
 }
 
 struct ConvGW {
@@ -960,8 +958,8 @@ GenPlan plan_gen(const ConvG &g, bool dx, bool va) {
 
 template <int WN, int NJ, int KW, bool DX>
 int launch_gen(const ConvG &g, const GenPlan &p, bool va) {
-  auto kern = va && !DX ? conv_gen_kernel<1, WN, 1, NJ, KW, DX, !DX>
-                        : conv_gen_kernel<1, WN, 1, NJ, KW, DX, false>;
+  auto kern = va && !DX ? conv_gen_kernel<WN, NJ, KW, DX, !DX>
+                        : conv_gen_kernel<WN, NJ, KW, DX, false>;
   if (p.lds > 64 * 1024 && !big_lds((const void *)kern)) return -1;
   const dim3 grid((unsigned)(p.ftiles * p.ptiles), 1, DX ? (unsigned)(g.sh * g.sw) : 1u);
   hipLaunchKernelGGL(kern, grid, dim3(NT), (size_t)p.lds, stream(), g);
