@@ -72,7 +72,7 @@ int tt_k_gemm_bias_ce(int M, int N, int K, const float *A, const float *B, const
                       float *rowloss, float scale);
 /* loss[0] = the mean of rowloss (rows floats) summed as
  * tt_k_softmax_ce_mean_hostlab sums its row losses (the loss of a
- * tt_k_gemm_bias_ce pass) */
+ * tt_k_gemm_bias_ce pass); past TT_CE_MEAN_MAX_ROWS rows over many workgroups */
 int tt_k_ce_mean_rows(const float *rowloss, float *loss, int rows);
 
 /* tt_k_gemm without any device allocation.  No counterpart in the

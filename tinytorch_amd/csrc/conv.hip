@@ -3259,9 +3259,10 @@ ConvCost conv_cost(const Geo &g, const int q[13], int what) {
   // / 205 us, and 1.0e-6 / 1.9e-7 from the 64-bit result)
   const bool tiled = what == 1 && g_dwt && plan_dwt(g, N).tg;
   const bool wide = tiled && (long)g.F * g.K >= 65536;
-  // Chunks are at least 8 channels: with fewer (of 316 forwards 18 were 10 %
-  // faster by chunks, 264 slower), 1x1 forwards of fewer than 32 (10 of 117, 87)
-  // and other 1x1 products (of 250 34, 151) stay too.
+  // Chunks are at least 8 channels: forwards and weight gradients of fewer (of 317
+  // forwards 18 were 10 % faster by chunks, 264 slower; of 316 weight gradients
+  // 58 and 152), 1x1 forwards of fewer than 32 (of 117 10 and 87) and the other
+  // 1x1 products (of 250 35 and 170) stay too.
   const bool one = g.HH * g.WW == 1;
   const bool keep = what == 0   ? g.C < 8 || (one && g.C < 32) ||
                                     (is_k3(g) && g.sh == 1 && g.sw == 1 &&
